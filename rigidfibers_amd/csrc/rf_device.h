@@ -102,6 +102,113 @@ struct FarQuad {
   }
 };
 
+// Far pairs.  When the centres of two fibers lie far enough apart, K(x_i + s t_i
+// - x_j - s' t_j) is, as a function of (s, s') on [-1, 1]^2, its tensor
+// interpolant in NP x NP Gauss-Legendre nodes to working accuracy, so every
+// projection sum_q w_q P_k(s_q) int P_m(s') K ds' of the pair follows from
+// NP x NP kernel values.  The weights carry the functionals themselves to the
+// nodes: the composite rule's (its own truncation included) as
+// sum_q w_q P_k(s_q) l_p(s_q) with the Lagrange basis l_p, the exact integral's
+// as w_p P_m(s_p) (zero for m >= NP, orthogonal to the interpolant).
+// np[0] nodes from r[0] on, np[1] between r[1] and r[0] (distances in units of
+// the fibers' half length): every projection k, m <= N then differs from the
+// composite (or exact) one by < 1e-8 of the largest G_0 component, in the worst
+// direction sampled, a tenth of the FP32 rounding of the kernel values.  A
+// coarser outer rule leaves more of its own truncation to reproduce and needs
+// the larger radii.
+struct FarRule {
+  int np[2];
+  double r[2];
+};
+__host__ __device__ constexpr FarRule far_rule(int N, int NQI) {
+  constexpr double fine[kMaxTerms + 1][2] = {{0, 0},     {3.7, 3.0}, {4.1, 3.2}, {4.7, 3.2}, {5.8, 3.6},
+                                             {7.6, 3.6}, {4.1, 3.3}, {4.5, 3.3}, {5.5, 3.4}};
+  constexpr double coarse[kMaxTerms + 1][2] = {{0, 0},     {4.6, 4.2}, {5.6, 4.4}, {5.6, 4.4}, {7.6, 5.0},
+                                               {7.6, 5.0}, {5.2, 3.7}, {5.2, 3.7}, {5.5, 3.7}};
+  FarRule f{};
+  f.np[0] = N <= 5 ? 6 : 8;
+  f.np[1] = N <= 5 ? 8 : 10;
+  for (int c = 0; c < 2; ++c) f.r[c] = NQI == 4 ? coarse[N][c] : fine[N][c];
+  return f;
+}
+
+// 0: the pair takes np[0] nodes, 1: np[1] nodes, -1: it is near.  d = x_i - x_j;
+// ti2, tj2 = |t|^2 of the two fibers (1, or what a caller's initial state has).
+// A non-finite distance is near.
+__device__ __forceinline__ int far_class(const FarRule& f, double dx, double dy, double dz, double ti2, double tj2) {
+  const double d2 = fma(dx, dx, fma(dy, dy, dz * dz));
+  const double u = fmax(1.0, fmax(ti2, tj2));
+  return d2 >= f.r[0] * f.r[0] * u ? 0 : (d2 >= f.r[1] * f.r[1] * u ? 1 : -1);
+}
+
+// Positive Gauss-Legendre nodes and weights of 6, 8 and 10 points.
+constexpr double kGL6Node[3] = {0.23861918608319690863, 0.66120938646626451366, 0.93246951420315202781};
+constexpr double kGL6Weight[3] = {0.46791393457269104739, 0.36076157304813860757, 0.17132449237917034504};
+constexpr double kGL10Node[5] = {0.14887433898163121089, 0.43339539412924719080, 0.67940956829902440623,
+                                 0.86506336668898451073, 0.97390652851717172008};
+constexpr double kGL10Weight[5] = {0.29552422471475287017, 0.26926671930999635509, 0.21908636251598204400,
+                                   0.14945134915058059315, 0.06667134430868813759};
+
+// The NP-point rule as the far pairs use it: positive nodes, and the weights
+// of P_0..P_N at them (at -s_h: (-1)^m of them) for the composite rule of NQI
+// intervals or, with exact, the integral over [-1, 1].
+__host__ __device__ constexpr double gl_node(int NP, int h) {
+  return NP == 6 ? kGL6Node[h] : (NP == 8 ? kGL8Node[h] : kGL10Node[h]);
+}
+__host__ __device__ constexpr double gl_weight(int NP, int h) {
+  return NP == 6 ? kGL6Weight[h] : (NP == 8 ? kGL8Weight[h] : kGL10Weight[h]);
+}
+// Rounding to FP32 must not leave a functional that is blind to constants
+// (even m >= 2) with a sum of its own: over thousands of sources of one sign
+// (the right-hand side's) that sum, 1e-8 of G_0 each, would add up.  So the
+// smallest weight of each mode absorbs the others' rounding: the even modes
+// then reproduce the functional of 1, the odd ones that of s.
+template <int N, int NP>
+struct FarWeights {
+  static constexpr int H = NP / 2;
+  float W[H][N + 1];
+  constexpr FarWeights() : W() {}
+  constexpr FarWeights(int NQI, bool exact) : W() {
+    double x[NP] = {}, acc[H][N + 1] = {};
+    for (int h = 0; h < H; ++h) {
+      x[h] = gl_node(NP, h);
+      x[H + h] = -x[h];
+    }
+    if (exact) {
+      for (int m = 0; m <= N; ++m)
+        for (int h = 0; h < H; ++h) acc[h][m] = m < NP ? gl_weight(NP, h) * legendre_value(m, x[h]) : 0.0;
+    } else {
+      const double gp[3] = {-kGaussNode, 0.0, kGaussNode};
+      const double gw[3] = {5.0 / 9.0, 8.0 / 9.0, 5.0 / 9.0};
+      for (int iv = 0; iv < NQI; ++iv)
+        for (int k = 0; k < 3; ++k) {
+          const double sq = -1.0 + (2.0 * iv + 1.0 + gp[k]) / NQI;
+          double P[N + 1] = {};
+          for (int m = 0; m <= N; ++m) P[m] = legendre_value(m, sq);
+          for (int h = 0; h < H; ++h) {
+            double l = gw[k] / NQI;  // w_q l_h(s_q)
+            for (int r = 0; r < NP; ++r)
+              if (r != h) l *= (sq - x[r]) / (x[h] - x[r]);
+            for (int m = 0; m <= N; ++m) acc[h][m] += l * P[m];
+          }
+        }
+    }
+    for (int m = 0; m <= N; ++m) {
+      int least = 0;
+      double sum = 0.0;  // the functional of 1 or s, less the rounded weights'
+      for (int h = 0; h < H; ++h) {
+        W[h][m] = static_cast<float>(acc[h][m]);
+        const double u = (m & 1) ? x[h] : 1.0;
+        sum += (acc[h][m] - static_cast<double>(W[h][m])) * u;
+        const double mag = acc[h][m] < 0.0 ? -acc[h][m] : acc[h][m];
+        const double low = acc[least][m] < 0.0 ? -acc[least][m] : acc[least][m];
+        if (mag < low) least = h;
+      }
+      W[least][m] = static_cast<float>(W[least][m] + sum / ((m & 1) ? x[least] : 1.0));
+    }
+  }
+};
+
 // Node s_q in FP64 and weight w_q in FP32 for a runtime node index (the
 // per-lane target node), computed exactly as Quad<> does.
 template <int NQI>
@@ -333,6 +440,25 @@ __device__ __forceinline__ void analytic_g(const NodeProducts& q, double eps2, c
 // Component index of the symmetric 3x3 pair (a, b) in (xx, yy, zz, xy, xz, yz).
 __host__ __device__ constexpr int sym_index(int a, int b) {
   return (a == b) ? a : ((a + b == 1) ? 3 : ((a + b == 2) ? 4 : 5));
+}
+
+// Scale of one (target, source) block of the FP16 copy from the bits of g,
+// the largest |projection| of the block's rows (modes m >= 1, projections
+// k >= 1): the first three components dot three of them with the unit t_i,
+// the others are projections themselves, so |T| <= sqrt(3) g < 2 g.  With g
+// = 1.f 2^(E - 127), sv = 2^(E - 140) > 2 g / 32768, so the stored values
+// T / sv stay below 32768 in magnitude (and dividing by a power of two is
+// exact); iv = 1 / sv.  An empty (or vanishing) block gets 0, 0; a
+// non-finite g is passed on as the scale.
+__device__ __forceinline__ void half_block_scale(unsigned gbits, float& sv, float& iv) {
+  const unsigned E = (gbits >> 23) & 0xffu;
+  if (E >= 14u && E < 255u) {
+    sv = __uint_as_float((E - 13u) << 23);
+    iv = __uint_as_float((267u - E) << 23);
+  } else {
+    sv = (E == 255u) ? __uint_as_float(gbits) : 0.0f;
+    iv = 0.0f;
+  }
 }
 
 }  // namespace rf

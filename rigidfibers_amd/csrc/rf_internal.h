@@ -33,6 +33,13 @@ hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double
 // (Theta_0 and Phi0 of every source mode) and the velocity constants
 // cpart[group][i][6] (cpart then holds max_pair_groups(M) * M * 6 doubles).
 PairGrid theta_grid(int M, int sources_per_iteration);
+// The far pairs (rf_far.hip): their sums go to the partial slots after the near
+// pairs' (slot0 on).
+PairGrid far_grid(int M);
+hipError_t launch_assemble_far(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
+                               const double* ori, float* T, double* bpart, int slot0, float* Tv, double* cpart,
+                               const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, _Float16* T16,
+                               float* S16);
 int64_t theta_stride(int M, int N);
 hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
                                  const double* ori, float* T, double* bpart, float* Tv, double* cpart,
@@ -146,6 +153,8 @@ hipError_t launch_gmres_control_batch(int ns, int m, int kdim, int nvb, double t
 hipError_t launch_orth_dots_batch(int nvb, int kdim, int phase, const SusDev* sus, const SusIter* it,
                                   const int2* vblocks, double* part, hipStream_t s);
 
+hipError_t launch_assemble_far_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
+                                     const int2* targets, const PhysConsts& pc, hipStream_t s);
 hipError_t launch_assemble_theta_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
                                        const int2* targets, const PhysConsts& pc, hipStream_t s);
 hipError_t launch_gemv_theta_batch(int N, int ntargets, const SusDev* sus, const SusIter* it, const int2* targets,
