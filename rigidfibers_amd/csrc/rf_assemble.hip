@@ -112,7 +112,7 @@ template <int N, int NQI, bool ANALYTIC>
 __global__ __launch_bounds__(kPairThreads) void assemble_kernel(int M, int64_t lda, const double* __restrict__ pos,
                                                                 const double* __restrict__ ori,
                                                                 float* __restrict__ A, double* __restrict__ bpart,
-                                                                int jgroup, PhysConsts pc) {
+                                                                int jgroup, PhysConsts pc, int jfirst, int jend) {
   constexpr Quad<N, NQI> quad{};
   constexpr int Q = 3 * NQI;
   constexpr int PAIRS = kPairThreads / Q;
@@ -129,8 +129,8 @@ __global__ __launch_bounds__(kPairThreads) void assemble_kernel(int M, int64_t l
   const int qi = tid - p * Q;
   const int i = blockIdx.x * PAIRS + p;
   const bool ivalid = i < M;
-  const int j0 = blockIdx.y * jgroup;
-  const int j1 = min(M, j0 + jgroup);
+  const int j0 = jfirst + blockIdx.y * jgroup;
+  const int j1 = min(jend, j0 + jgroup);
   const int64_t n = static_cast<int64_t>(ROWS) * M;
 
   double xi[3] = {0, 0, 0}, tid_[3] = {0, 0, 0};
@@ -220,7 +220,7 @@ __global__ __launch_bounds__(kPairThreads) void assemble_kernel(int M, int64_t l
         continue;
       }
       const int kj = m - 1;
-      const int64_t col = static_cast<int64_t>(ROWS) * j + 3 * kj + bcol;
+      const int64_t col = static_cast<int64_t>(ROWS) * (j - jfirst) + 3 * kj + bcol;
       float* out = A + col * lda + static_cast<int64_t>(ROWS) * i2;
       if (i2 == j) {
 #pragma unroll
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kPairThreads) void assemble_kernel(int M, int64_t l
     __syncthreads();
   }
 
-  if (tid < PAIRS) {
+  if (tid < PAIRS && bpart != nullptr) {
     const int i2 = blockIdx.x * PAIRS + tid;
     if (i2 < M) {
       double* dst = bpart + static_cast<int64_t>(blockIdx.y) * n + static_cast<int64_t>(ROWS) * i2;
@@ -323,7 +323,7 @@ typedef float floatx2 __attribute__((ext_vector_type(2)));
 // A suspension has few near sources (8 of 5000 in a ball at 0.028 fibers per
 // unit volume, about 20 at 0.1), so the sweeps are few and the scan, one
 // distance per source, is most of the launch.
-template <int N, int NQI, bool ANALYTIC, bool HALF = false>
+template <int N, int NQI, bool ANALYTIC, bool HALF = false, bool SEGMENTS = false>
 __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_t Lp, bool all,
                                                     const double* __restrict__ pos,
                                                     const double* __restrict__ ori, float* __restrict__ T,
@@ -332,7 +332,8 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
                                                     const double* __restrict__ x0, double* __restrict__ apart,
                                                     _Float16* __restrict__ T16 = nullptr,
                                                     float* __restrict__ S16 = nullptr,
-                                                    const SusDev* __restrict__ serving = nullptr) {
+                                                    const SusDev* __restrict__ serving = nullptr,
+                                                    const NearStore* __restrict__ store = nullptr) {
   constexpr Quad<N, NQI> quad{};
   constexpr FarRule rule = far_rule(N, NQI);
   constexpr int Q = 3 * NQI;
@@ -372,11 +373,48 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
   const double ti2 = fma(tid_[2], tid_[2], fma(tid_[1], tid_[1], tid_[0] * tid_[0]));
   const double sq_d = node_fp64<NQI>(qi);
   const float sq = static_cast<float>(sq_d);
-  float* Ti = T + static_cast<int64_t>(i) * NC * Lp;
+  float* Ti = SEGMENTS ? nullptr : T + static_cast<int64_t>(i) * NC * Lp;
   float* Vi = Tv ? Tv + static_cast<int64_t>(i) * 12 * Lp : nullptr;
   _Float16* const Hi = HALF ? T16 + static_cast<int64_t>(i) * NC * Lp : nullptr;
   if (serving != nullptr) x0 = serving->x0;
-  const uint32_t lp32 = static_cast<uint32_t>(Lp);
+  uint32_t lp32 = static_cast<uint32_t>(Lp);
+  auto is_near = [&](int j) {
+    if (j >= je || j == i) return false;
+    if (all) return true;
+    const double t0 = ori[3 * j], t1 = ori[3 * j + 1], t2 = ori[3 * j + 2];
+    const int c = far_class(rule, xi[0] - pos[3 * j], xi[1] - pos[3 * j + 1], xi[2] - pos[3 * j + 2], ti2,
+                            fma(t2, t2, fma(t1, t1, t0 * t0)));
+    return SEGMENTS ? c != 0 : c < 0;
+  };
+  // The target's segment: counted, then taken from the store.  Where it starts
+  // depends on the order the workgroups come in, what it holds does not.
+  int* seg = nullptr;  // its sources
+  int formed = 0;      // pairs of the segment formed so far
+  if constexpr (SEGMENTS) {
+    __shared__ long long seg_base;
+    int mine = 0;
+    for (int j = jb + tid; j < je; j += kPairThreads) mine += is_near(j) ? 1 : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
+    if (lane == 0) ncount[0][wave] = mine;
+    __syncthreads();
+    int cnt = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) cnt += ncount[0][w];
+    lp32 = static_cast<uint32_t>(near_stride(cnt, N));
+    if (tid == 0) {
+      const int64_t size = near_ints(cnt) + static_cast<int64_t>(NC + (store->velocity ? 12 : 0)) * lp32;
+      const int64_t at = static_cast<int64_t>(atomicAdd(store->used, static_cast<unsigned long long>(size)));
+      seg_base = at + size <= store->capacity ? at : -1;
+      store->base[i] = seg_base;
+      store->count[i] = cnt;
+    }
+    __syncthreads();
+    if (seg_base < 0) return;  // no room: the host takes more and repeats the launch
+    seg = reinterpret_cast<int*>(store->data + seg_base);
+    Ti = store->data + seg_base + near_ints(cnt);
+    Vi = store->velocity ? Ti + static_cast<int64_t>(NC) * lp32 : nullptr;
+  }
 
   // RHS (and velocity-constant) and product sums of each source slot, kept in
   // LDS; the mode factors gamma_k, eigen_k as a table the lanes index by k
@@ -389,7 +427,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       modes[kMaxTerms + t] = pc.eigen[t];
     }
   // the self pair
-  if (i >= jb && i < je) {
+  if (!SEGMENTS && i >= jb && i < je) {
     const uint32_t col = static_cast<uint32_t>(i) * N;
     for (int r = tid; r < NC * N; r += kPairThreads) {
       const uint32_t u = r / N, k = r - (r / N) * N;
@@ -413,15 +451,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
     int before[kPer];
 #pragma unroll
     for (int t = 0; t < kPer; ++t) {
-      const int j = js + t * kPairThreads + tid;
-      near[t] = false;
-      if (all) {
-        near[t] = j < je && j != i;
-      } else if (j < je && j != i) {
-        const double t0 = ori[3 * j], t1 = ori[3 * j + 1], t2 = ori[3 * j + 2];
-        near[t] = far_class(rule, xi[0] - pos[3 * j], xi[1] - pos[3 * j + 1], xi[2] - pos[3 * j + 2], ti2,
-                            fma(t2, t2, fma(t1, t1, t0 * t0))) < 0;
-      }
+      near[t] = is_near(js + t * kPairThreads + tid);
       const unsigned long long mask = __ballot(near[t]);
       before[t] = __builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(mask >> 32),
                                             __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(mask), 0u));
@@ -444,6 +474,11 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       const int take = min(pend, PAIRS);
       pend -= take;
       const int* const js_ = nlist + pend;  // this sweep's sources
+      // first column of source slot q
+      auto col0 = [&](int q) { return SEGMENTS ? (formed + q) * N : js_[q] * N; };
+      if constexpr (SEGMENTS) {
+        if (tid < take) seg[formed + tid] = js_[tid];
+      }
       if (tid < PAIRS) smax[tid] = 0u;
       if (p < take) {
         const int j = js_[p];
@@ -502,7 +537,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
         const int u = job / PN, pm = job - u * PN, s = pm / N;
         if (s >= take) continue;
         const float val = sys_val(u, pm);
-        const uint32_t at = static_cast<uint32_t>(u) * lp32 + static_cast<uint32_t>(js_[s] * N + (pm - s * N));
+        const uint32_t at = static_cast<uint32_t>(u) * lp32 + static_cast<uint32_t>(col0(s) + (pm - s * N));
         Ti[at] = val;
         if constexpr (HALF) {
           float sv, iv;
@@ -517,7 +552,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
           if (s >= take) continue;
           const int kk = w < 6 ? 1 : 0;
           const int c = w < 6 ? w : w - 6;
-          Vi[static_cast<uint32_t>(w) * lp32 + static_cast<uint32_t>(js_[s] * N + (pm - s * N))] =
+          Vi[static_cast<uint32_t>(w) * lp32 + static_cast<uint32_t>(col0(s) + (pm - s * N))] =
               Pj[kk * RP + c * CB + PAIRS + pm];
         }
       }
@@ -579,13 +614,14 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
         }
       }
       __syncthreads();  // the sweep's LDS is free
+      if constexpr (SEGMENTS) formed += take;
     }
     if (last) break;
   }
 
   // Row tid of b, of the off-diagonal product A x0, and the velocity constants:
   // the slots' sums in order.  Serving adds the far pairs' sums, which the far
-  // kernel left in b, cpart and V_0.
+  // kernel left in b, cpart and V_0 (unless every pair is near).
   auto slots = [&](const double* first, int stride) {
     double s = 0.0;
     for (int q = 0; q < PAIRS; ++q) s += first[q * stride];
@@ -610,13 +646,13 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       bpart[static_cast<int64_t>(gy) * n + row] = sb;
       if (apart && x0 != nullptr) apart[static_cast<int64_t>(gy) * n + row] = out;
     } else {
-      sb += bpart[row];
+      if (!all) sb += bpart[row];
       bpart[row] = sb;
     }
   } else if (cpart && tid < NR) {
     double s = slots(&bred[0][tid], NR);
     double* c = cpart + (static_cast<int64_t>(gy) * M + i) * 6 + (tid - ROWS);
-    if (serving != nullptr) s += *c;
+    if (serving != nullptr && !all) s += *c;
     *c = s;
   }
   // Serving (all sources in this workgroup): the first residual r0 = b - (x0 +
@@ -627,7 +663,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
     double* nred = reinterpret_cast<double*>(Pj);  // Pj is free after the last sweep
     double* const r0v = serving->V;
     if (tid < ROWS) {
-      const double r = (x0 != nullptr) ? sb - (out + r0v[row] + x0[row]) : sb;
+      const double r = (x0 != nullptr) ? sb - ((all ? out : out + r0v[row]) + x0[row]) : sb;
       r0v[row] = r;
       nred[tid] = sb * sb;
       nred[ROWS + tid] = r * r;
@@ -668,6 +704,17 @@ __global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(th
                                                cpart, x0, apart, T16, S16);
 }
 
+// The pairs of a large suspension that a product does not form again: workgroup
+// = target fiber, every source.
+template <int N, int NQI, bool ANALYTIC>
+__global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(theta_min_waves<N, NQI, ANALYTIC>(), 8))) void assemble_segments_kernel(
+    int M, const double* __restrict__ pos, const double* __restrict__ ori, NearStore store,
+    double* __restrict__ bpart, PhysConsts pc, double* __restrict__ cpart, const double* __restrict__ x0,
+    double* __restrict__ apart) {
+  assemble_near_block<N, NQI, ANALYTIC, false, true>(blockIdx.x, 0, M, 0, false, pos, ori, nullptr, bpart, M, pc,
+                                                     nullptr, cpart, x0, apart, nullptr, nullptr, nullptr, &store);
+}
+
 // Serving: workgroup = (suspension, target fiber), all sources in one group;
 // after the far kernel, so b and the velocity constants are complete here, and
 // with them the first GMRES residual (into the basis' first vector) and its
@@ -677,7 +724,7 @@ __global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(th
     const SusDev* __restrict__ sus, const int2* __restrict__ targets, PhysConsts pc) {
   const int2 e = targets[blockIdx.x];
   const SusDev& d = sus[e.x];
-  assemble_near_block<N, NQI, ANALYTIC>(e.y, 0, d.M, d.Lp, false, d.pos, d.ori, d.T, d.b, d.M, pc, d.Tv, d.cpart, nullptr,
+  assemble_near_block<N, NQI, ANALYTIC>(e.y, 0, d.M, d.Lp, d.M < far_min_fibers(ANALYTIC), d.pos, d.ori, d.T, d.b, d.M, pc, d.Tv, d.cpart, nullptr,
                                          nullptr, nullptr, nullptr, &d);
 }
 
@@ -786,32 +833,34 @@ int64_t theta_stride(int M, int N) { return (static_cast<int64_t>(M) * N + 63) /
 
 template <int N, int NQI, bool AN>
 static hipError_t launch_asm_t(int M, int64_t lda, const double* pos, const double* ori, float* A, double* bpart,
-                               const PhysConsts& pc, hipStream_t s) {
+                               const PhysConsts& pc, hipStream_t s, int j0, int jcount) {
   constexpr int PAIRS = kPairThreads / (3 * NQI);
-  const PairGrid g = pair_grid(M, PAIRS);
+  PairGrid g = pair_grid(M, PAIRS);
+  if (bpart == nullptr) g.groups = (jcount + g.jgroup - 1) / g.jgroup;
   hipLaunchKernelGGL((assemble_kernel<N, NQI, AN>), dim3(g.tiles, g.groups), dim3(kPairThreads), 0, s, M, lda, pos,
-                     ori, A, bpart, g.jgroup, pc);
+                     ori, A, bpart, g.jgroup, pc, j0, j0 + jcount);
   return hipGetLastError();
 }
 
 template <int N, int NQI>
 static hipError_t launch_asm_n(bool an, int M, int64_t lda, const double* pos, const double* ori, float* A,
-                               double* bpart, const PhysConsts& pc, hipStream_t s) {
-  return an ? launch_asm_t<N, NQI, true>(M, lda, pos, ori, A, bpart, pc, s)
-            : launch_asm_t<N, NQI, false>(M, lda, pos, ori, A, bpart, pc, s);
+                               double* bpart, const PhysConsts& pc, hipStream_t s, int j0, int jcount) {
+  return an ? launch_asm_t<N, NQI, true>(M, lda, pos, ori, A, bpart, pc, s, j0, jcount)
+            : launch_asm_t<N, NQI, false>(M, lda, pos, ori, A, bpart, pc, s, j0, jcount);
 }
 
 bool assemble_supported(int N, int NQI) { return N >= 1 && N <= kMaxTerms && (NQI == 4 || NQI == 8 || NQI == 16); }
 
 #define RF_ASM_CASE(NN)                                                                      \
   case NN:                                                                                   \
-    if (NQI == 4) return launch_asm_n<NN, 4>(analytical, M, lda, pos, ori, A, bpart, pc, s); \
-    if (NQI == 8) return launch_asm_n<NN, 8>(analytical, M, lda, pos, ori, A, bpart, pc, s); \
-    if (NQI == 16) return launch_asm_n<NN, 16>(analytical, M, lda, pos, ori, A, bpart, pc, s); \
+    if (NQI == 4) return launch_asm_n<NN, 4>(analytical, M, lda, pos, ori, A, bpart, pc, s, j0, jcount); \
+    if (NQI == 8) return launch_asm_n<NN, 8>(analytical, M, lda, pos, ori, A, bpart, pc, s, j0, jcount); \
+    if (NQI == 16) return launch_asm_n<NN, 16>(analytical, M, lda, pos, ori, A, bpart, pc, s, j0, jcount); \
     return hipErrorInvalidValue;
 
-hipError_t launch_assemble(int N, int NQI, bool analytical, int M, int64_t lda, const double* pos,
-                           const double* ori, float* A, double* bpart, const PhysConsts& pc, hipStream_t s) {
+static hipError_t launch_asm(int N, int NQI, bool analytical, int M, int64_t lda, const double* pos,
+                             const double* ori, float* A, double* bpart, const PhysConsts& pc, hipStream_t s, int j0,
+                             int jcount) {
   switch (N) {
     RF_ASM_CASE(1)
     RF_ASM_CASE(2)
@@ -827,13 +876,17 @@ hipError_t launch_assemble(int N, int NQI, bool analytical, int M, int64_t lda, 
 }
 #undef RF_ASM_CASE
 
-// Below this many fibers every pair takes the near kernel alone: the launch is
-// then its latency, and the far kernel's own (24 us at M = 100: a few wavefronts
-// with one batch after another) is longer than what it takes off the near one's.
-// Assembly in us, near alone / with the far kernel, at 0.1 fibers per unit
-// volume: numerical M = 200 78 / 84, 250 107 / 95, 400 187 / 126; analytical
-// 300 103 / 124, 400 140 / 131, 600 243 / 196.
-constexpr int far_min_fibers(bool analytical) { return analytical ? 384 : 240; }
+hipError_t launch_assemble(int N, int NQI, bool analytical, int M, int64_t lda, const double* pos,
+                           const double* ori, float* A, double* bpart, const PhysConsts& pc, hipStream_t s) {
+  return launch_asm(N, NQI, analytical, M, lda, pos, ori, A, bpart, pc, s, 0, M);
+}
+
+hipError_t launch_assemble_columns(int N, int NQI, bool analytical, int M, int64_t lda, const double* pos,
+                                   const double* ori, float* A, const PhysConsts& pc, hipStream_t s, int j0,
+                                   int jcount) {
+  if (j0 < 0 || jcount < 1 || j0 + jcount > M) return hipErrorInvalidValue;
+  return launch_asm(N, NQI, analytical, M, lda, pos, ori, A, nullptr, pc, s, j0, jcount);
+}
 
 template <int N, int NQI, bool AN>
 static hipError_t launch_theta_t(int M, int64_t Lp, const double* pos, const double* ori, float* T, double* bpart,
@@ -891,6 +944,41 @@ hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t
   }
 }
 #undef RF_TH_CASE
+
+hipError_t launch_assemble_near(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
+                                const NearStore& near, double* bpart, double* cpart, const double* x0, double* apart,
+                                const PhysConsts& pc, hipStream_t s) {
+  const dim3 grid(M), block(kPairThreads);
+#define RF_SEG(NN, QQ)                                                                                              \
+  if (NQI == QQ) {                                                                                                  \
+    if (analytical)                                                                                                 \
+      hipLaunchKernelGGL((assemble_segments_kernel<NN, QQ, true>), grid, block, 0, s, M, pos, ori, near, bpart, pc,  \
+                         cpart, x0, apart);                                                                         \
+    else                                                                                                            \
+      hipLaunchKernelGGL((assemble_segments_kernel<NN, QQ, false>), grid, block, 0, s, M, pos, ori, near, bpart, pc, \
+                         cpart, x0, apart);                                                                         \
+    return hipGetLastError();                                                                                       \
+  }
+#define RF_SEG_N(NN) \
+  case NN:           \
+    RF_SEG(NN, 4)    \
+    RF_SEG(NN, 8)    \
+    RF_SEG(NN, 16)   \
+    break;
+  switch (N) {
+    RF_SEG_N(1)
+    RF_SEG_N(2)
+    RF_SEG_N(3)
+    RF_SEG_N(4)
+    RF_SEG_N(5)
+    RF_SEG_N(6)
+    RF_SEG_N(7)
+    RF_SEG_N(8)
+  }
+#undef RF_SEG_N
+#undef RF_SEG
+  return hipErrorInvalidValue;
+}
 
 // The whole dense A from the theta form, for the LU's factor storage
 // (leading dimension lda), with the arithmetic of expand_theta_kernel (the

@@ -88,6 +88,10 @@ struct rf_simulation {
   int tori = 0;
   bool tori_valid = false;
   int64_t Lp = 0;         // theta component stride
+  bool oper = false;      // iterative solvers, large: products from the near pairs and the state (rf_operator.hip)
+  rf::Operator op{};
+  unsigned long long* near_used = nullptr;  // op.near.used mirrored into pinned host memory
+  hipEvent_t near_done = nullptr;
   int bgroups = 1;        // RHS partial slots written by the last assembly
   bool vstored = false;   // the theta assembly also stores the velocity operator
   bool vvalid = false;    // ... and it belongs to the current state
@@ -258,6 +262,9 @@ hipError_t sim_gemv(rf_simulation* s, const double* x, double* part, double* y, 
     e1 = s->gev[2 * s->ngemv + 1];
     ++s->ngemv;
   }
+  if (s->oper)
+    return rf::op_product(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, x, y, b, mode,
+                          s->pc, s->stream, e0, e1, skip);
   if (s->theta)
     return rf::gemv_theta(s->N, s->M, s->Lp, s->T, s->ori[s->cur], x, y, b, mode, s->pc, s->stream, e0, e1, skip);
   return rf::gemv(s->plan, s->A, x, part, y, b, mode, s->stream, e0, e1, skip);
@@ -520,7 +527,10 @@ rf_status solve_bicgstab(rf_simulation* s) {
     RF_HIP(rf::bicg_start(s->bicg, rho, res, s->stream));
     for (int k = 0; k < maxit; ++k) {
       if (k > 0) {  // a pending restart: r = b - A x (untimed), r0 = p = r, rho = ||r||^2
-        if (s->theta)
+        if (s->oper)
+          RF_HIP(rf::op_product(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->x, r,
+                                s->b, 1, s->pc, s->stream, nullptr, nullptr, &s->bicg.head->no_restart));
+        else if (s->theta)
           RF_HIP(rf::gemv_theta(s->N, s->M, s->Lp, s->T, s->ori[s->cur], s->x, r, s->b, 1, s->pc, s->stream,
                                 nullptr, nullptr, &s->bicg.head->no_restart));
         else
@@ -603,6 +613,53 @@ rf_status solve_direct(rf_simulation* s) {
   s->stats.relative_residual = st.relative_residual;
   s->stats.converged = st.converged;
   if (!std::isfinite(st.relative_residual)) return fail(RF_ERR_NONFINITE, "non-finite solution in the direct solve");
+  return RF_OK;
+}
+
+// Room for the operator's stored pairs: at least `floats`, in place of what
+// there is (which nothing in flight may use).
+rf_status near_reserve(rf_simulation* s, int64_t floats) {
+  rf::NearStore& near = s->op.near;
+  if (near.data) (void)hipFree(near.data);
+  s->device_bytes -= near.capacity * static_cast<int64_t>(sizeof(float));
+  near.data = nullptr;
+  near.capacity = 0;
+  void* q = nullptr;
+  const hipError_t e = hipMalloc(&q, static_cast<size_t>(floats) * sizeof(float));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(RF_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(floats * 4) + " bytes for the near pairs failed: " +
+                                          hipGetErrorString(e));
+  }
+  near.data = static_cast<float*>(q);
+  near.capacity = floats;
+  s->device_bytes += floats * static_cast<int64_t>(sizeof(float));
+  return RF_OK;
+}
+
+// The operator's assembly: the near pairs into their store, the far pairs'
+// sums beside them.  How much the near pairs take is known only when they have
+// been counted: the launch that finds too little room says how much it needs,
+// the store grows by a quarter more than that and the launch is repeated.
+rf_status assemble_operator(rf_simulation* s, const double* x0) {
+  double* const apart = x0 ? s->apart : nullptr;
+  double* const cpart = s->vstored ? s->cpart : nullptr;
+  for (int attempt = 0;; ++attempt) {
+    RF_HIP(rf::fill(1, 0.0, reinterpret_cast<double*>(s->op.near.used), s->stream));
+    RF_HIP(rf::launch_assemble_near(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op.near,
+                                    s->bpart, cpart, x0, apart, s->pc, s->stream));
+    RF_HIP(hipMemcpyAsync(s->near_used, s->op.near.used, sizeof(*s->near_used), hipMemcpyDeviceToHost, s->stream));
+    RF_HIP(hipEventRecord(s->near_done, s->stream));
+    if (attempt == 0)  // on the GPU while the host waits for the count
+      RF_HIP(rf::op_assemble_far(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->bpart,
+                                 cpart, x0, apart, s->pc, s->stream));
+    RF_HIP(hipEventSynchronize(s->near_done));
+    const int64_t used = static_cast<int64_t>(*static_cast<volatile unsigned long long*>(s->near_used));
+    if (used <= s->op.near.capacity) break;
+    RF_HIP(hipStreamSynchronize(s->stream));
+    RF_TRY(near_reserve(s, used + used / 4));
+  }
+  s->bgroups = 2;
   return RF_OK;
 }
 
@@ -756,7 +813,32 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
   // The theta form unless the dense one is asked for: the direct solvers
   // expand it into their factor storage and refine with the theta GEMV.
   s->theta = cfg->matrix_format != RF_MATRIX_DENSE;
-  if (s->theta) {
+  // Large suspensions of the iterative solvers: the far pairs' values are formed
+  // again in each product instead of being stored (0.70 against 2.05 ms a product
+  // at M = 5000, and the assembly has only the other pairs to form).
+  s->oper = cfg->matrix_format == RF_MATRIX_AUTO && iterative && cfg->solver != RF_SOLVER_GMRES_IR &&
+            rf::operator_form(M, s->N);
+  if (s->oper) {
+    s->theta = false;
+    s->vstored = cfg->velocity_operator == RF_VELOCITY_STORED && s->vel_analytical == s->analytical;
+    if (s->vstored && st == RF_OK)
+      st = s->alloc(&s->cpart, static_cast<size_t>(rf::max_pair_groups(M)) * M * 6);
+    double* used = nullptr;
+    if (st == RF_OK) st = s->alloc(&used, 1);
+    s->op.near.used = reinterpret_cast<unsigned long long*>(used);
+    if (st == RF_OK) st = s->alloc(&s->op.near.base, static_cast<size_t>(M));
+    if (st == RF_OK) st = s->alloc(&s->op.near.count, static_cast<size_t>(M));
+    s->op.near.velocity = s->vstored ? 1 : 0;
+    if (st == RF_OK) st = s->alloc(&s->op.nodes, rf::op_node_doubles(M, s->N));
+    if (st == RF_OK) st = s->alloc(&s->op.part, rf::op_part_doubles(M, s->N));
+    // 96 near sources per target to begin with (46 in a ball of 5000 fibers at
+    // 0.028 per unit volume, about 180 at 0.1)
+    if (st == RF_OK)
+      st = near_reserve(s, static_cast<int64_t>(M) * (96 + (3 + 6 * (s->N - 1) + (s->vstored ? 12 : 0)) *
+                                                               rf::near_stride(96, s->N)));
+    if (st == RF_OK && hipEventCreateWithFlags(&s->near_done, hipEventDisableTiming) != hipSuccess)
+      st = fail(RF_ERR_DEVICE, "hipEventCreate failed");
+  } else if (s->theta) {
     const int NC = 3 + 6 * (s->N - 1);
     s->Lp = rf::theta_stride(M, s->N);
     if (st == RF_OK) st = s->alloc(&s->T, static_cast<size_t>(M) * NC * static_cast<size_t>(s->Lp));
@@ -775,7 +857,7 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
   if (st == RF_OK) st = s->alloc(&s->x, static_cast<size_t>(n));
   if (st == RF_OK && cfg->initial_guess == RF_GUESS_EXTRAPOLATED) st = s->alloc(&s->xprev, static_cast<size_t>(n));
   if (st == RF_OK) st = s->alloc(&s->bpart, static_cast<size_t>(rf::max_pair_groups(M)) * n);
-  if (s->theta && iterative && !cfg->separate_residual) {
+  if ((s->theta || s->oper) && iterative && !cfg->separate_residual) {
     if (st == RF_OK) st = s->alloc(&s->apart, static_cast<size_t>(rf::max_pair_groups(M)) * n);
     if (st == RF_OK) st = s->alloc(&s->r0, static_cast<size_t>(n));
   }
@@ -812,6 +894,7 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
       st = fail(RF_ERR_OUT_OF_MEMORY, "hipHostMalloc of the solver's done flag failed");
     } else if (st == RF_OK) {
       s->hdone = static_cast<int*>(hp);
+      s->near_used = static_cast<unsigned long long*>(hp) + 2;
       *s->hdone = 0;
       s->cyc.hdone = static_cast<int*>(dp);
       s->bicg.hdone = static_cast<int*>(dp);
@@ -849,6 +932,8 @@ void rf_destroy(rf_simulation* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   rf::lu_workspace_destroy(&s->lu);
   for (void* p : s->allocations) (void)hipFree(p);
+  if (s->op.near.data) (void)hipFree(s->op.near.data);
+  if (s->near_done) (void)hipEventDestroy(s->near_done);
   for (auto& e : s->ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : s->gev)
@@ -866,7 +951,7 @@ rf_status rf_assemble_system(rf_simulation* s) {
   if (!s) return fail(RF_ERR_INVALID_ARGUMENT, "simulation is NULL");
   const double* x0 = nullptr;
   s->r0_ready = false;
-  if (s->theta) {
+  if (s->theta || s->oper) {
     if (s->apart) {  // the solve's initial guess now, its residual with the system
       if (!s->guess_taken) {
         bool warm = false;
@@ -877,7 +962,10 @@ rf_status rf_assemble_system(rf_simulation* s) {
       if (s->guess_warm) x0 = s->x;
     }
     RF_HIP(hipEventRecord(s->ev[5], s->stream));
-    RF_HIP(rf::launch_assemble_theta(s->N, s->NQI, s->analytical, s->M, s->Lp, s->pos[s->cur], s->ori[s->cur], s->T,
+    if (s->oper)
+      RF_TRY(assemble_operator(s, x0));
+    else
+      RF_HIP(rf::launch_assemble_theta(s->N, s->NQI, s->analytical, s->M, s->Lp, s->pos[s->cur], s->ori[s->cur], s->T,
                                      s->bpart, s->Tv, s->cpart, x0, x0 ? s->apart : nullptr, s->pc, s->stream,
                                      &s->bgroups, s->T16, s->S16));
     RF_HIP(hipEventRecord(s->ev[6], s->stream));
@@ -924,7 +1012,10 @@ rf_status rf_solve_system(rf_simulation* s) {
 
 rf_status rf_update_velocities(rf_simulation* s) {
   if (!s) return fail(RF_ERR_INVALID_ARGUMENT, "simulation is NULL");
-  if (s->vstored && s->vvalid)
+  if (s->oper && s->vstored && s->vvalid)
+    RF_HIP(rf::op_velocities(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->cpart, s->x,
+                             s->pc, s->tv[s->vcur], s->rv[s->vcur], s->stream));
+  else if (s->vstored && s->vvalid)
     RF_HIP(rf::launch_velocities_stored(s->N, s->M, s->Lp, s->Tv, s->cpart, s->bgroups, s->ori[s->cur], s->x, s->pc,
                                         s->tv[s->vcur], s->rv[s->vcur], s->stream));
   else
@@ -1055,10 +1146,10 @@ rf_status rf_set_state(rf_simulation* s, const double* positions, const double* 
 rf_status rf_get_system(rf_simulation* s, float* a_matrix, double* b_vector, double* x_vector) {
   if (!s) return fail(RF_ERR_INVALID_ARGUMENT, "simulation is NULL");
   const int64_t n = s->n;
-  if (a_matrix && s->theta && !s->tori_valid)
+  if (a_matrix && (s->theta || s->oper) && !s->tori_valid)
     return fail(RF_ERR_INVALID_ARGUMENT, "no theta-form system to expand (none assembled, or the state it was "
                                          "assembled from has been overwritten)");
-  if (a_matrix && s->theta) {
+  if (a_matrix && (s->theta || s->oper)) {
     // rebuild the dense blocks in a temporary device buffer
     float* tmp = nullptr;
     hipError_t e = hipMalloc(&tmp, sizeof(float) * static_cast<size_t>(n) * static_cast<size_t>(n));
@@ -1066,7 +1157,9 @@ rf_status rf_get_system(rf_simulation* s, float* a_matrix, double* b_vector, dou
       (void)hipGetLastError();
       return fail(RF_ERR_OUT_OF_MEMORY, "no device memory to expand the theta-form matrix");
     }
-    e = rf::launch_expand_theta(s->N, s->M, s->Lp, s->T, s->ori[s->tori], s->pc, tmp, s->stream);
+    e = s->oper ? rf::launch_assemble_columns(s->N, s->NQI, s->analytical, s->M, n, s->pos[s->tori], s->ori[s->tori],
+                                              tmp, s->pc, s->stream, 0, s->M)
+                : rf::launch_expand_theta(s->N, s->M, s->Lp, s->T, s->ori[s->tori], s->pc, tmp, s->stream);
     if (e == hipSuccess)
       e = hipMemcpyAsync(a_matrix, tmp, sizeof(float) * static_cast<size_t>(n) * n, hipMemcpyDeviceToHost, s->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
@@ -1084,7 +1177,7 @@ rf_status rf_get_system(rf_simulation* s, float* a_matrix, double* b_vector, dou
 
 rf_status rf_get_system_noalloc(rf_simulation* s, float* a_matrix, double* b_vector, double* x_vector) {
   if (!s) return fail(RF_ERR_INVALID_ARGUMENT, "simulation is NULL");
-  if (!a_matrix || !s->theta) return rf_get_system(s, a_matrix, b_vector, x_vector);  // no staging needed
+  if (!a_matrix || !(s->theta || s->oper)) return rf_get_system(s, a_matrix, b_vector, x_vector);  // no staging needed
   if (!s->tori_valid)
     return fail(RF_ERR_INVALID_ARGUMENT, "no theta-form system to expand (none assembled, or the state it was "
                                          "assembled from has been overwritten)");
@@ -1102,7 +1195,11 @@ rf_status rf_get_system_noalloc(rf_simulation* s, float* a_matrix, double* b_vec
   // the expansion writes every element of a chunk, so nothing is cleared.
   for (int j0 = 0; j0 < s->M; j0 += chunk) {
     const int jc = std::min(chunk, s->M - j0);
-    RF_HIP(rf::launch_expand_theta(s->N, s->M, s->Lp, s->T, s->ori[s->tori], s->pc, stage, s->stream, j0, jc));
+    if (s->oper)
+      RF_HIP(rf::launch_assemble_columns(s->N, s->NQI, s->analytical, s->M, s->n, s->pos[s->tori], s->ori[s->tori],
+                                         stage, s->pc, s->stream, j0, jc));
+    else
+      RF_HIP(rf::launch_expand_theta(s->N, s->M, s->Lp, s->T, s->ori[s->tori], s->pc, stage, s->stream, j0, jc));
     RF_HIP(hipMemcpyAsync(a_matrix + static_cast<int64_t>(j0) * fiber_cols, stage,
                           sizeof(float) * static_cast<size_t>(jc) * static_cast<size_t>(fiber_cols),
                           hipMemcpyDeviceToHost, s->stream));

@@ -46,6 +46,35 @@ __host__ __device__ constexpr double legendre_value(int f, double s) {
   return acc;
 }
 
+// Rounds the H weights of one mode, at the nodes +s (those at -s are +- the
+// same), to Real.  Rounding must not leave a functional that is blind to
+// constants (even m >= 2) with a sum of its own: over thousands of sources of
+// one sign (the right-hand side's) that sum, 1e-8 of G_0 each, would add up.
+// So the rounded weights reproduce the exact ones' functional of 1 (even m) or
+// of s (odd m): from the largest weight to the smallest, each takes up the
+// rounding of those before it, which moves no weight by more than an ulp or so.
+template <class Real, int H>
+__host__ __device__ constexpr void round_weights(const double (&exact)[H], const double (&s)[H], bool odd,
+                                                 Real (&out)[H]) {
+  bool done[H] = {};
+  double left = 0.0;
+  for (int n = 0; n < H; ++n) {
+    int q = -1;
+    for (int k = 0; k < H; ++k) {
+      const double a = exact[k] < 0.0 ? -exact[k] : exact[k];
+      if (!done[k] && (q < 0 || a > (exact[q] < 0.0 ? -exact[q] : exact[q]))) q = k;
+    }
+    done[q] = true;
+    const double u = odd ? s[q] : 1.0;
+    // within an ulp: the lever of a node near the centre on s is short
+    double add = left / u;
+    const double most = 1.2e-7 * (exact[q] < 0.0 ? -exact[q] : exact[q]);
+    add = add > most ? most : (add < -most ? -most : add);
+    out[q] = static_cast<Real>(exact[q] + (sizeof(Real) < sizeof(double) ? add : 0.0));
+    left += (exact[q] - static_cast<double>(out[q])) * u;
+  }
+}
+
 // Composite 3-point Gauss-Legendre rule on NQI equal intervals of [-1, 1] and
 // the weighted Legendre table W[m][q] = w_q * P_m(s_q), m = 0..N.
 template <int N, int NQI>
@@ -74,6 +103,23 @@ struct Quad {
         P[m][q] = static_cast<float>(legendre_value(m, sd[q]));
         W[m][q] = w[q] * P[m][q];
       }
+    // W[m][Q-1-q] = (-1)^m W[m][q].  Modes 0 and 1 keep the products of the
+    // rounded tables, which the pairwise velocities take.  b's error against FP64
+    // went from 1.7 - 3.5e-6 to 0.4 - 1.6e-6 of its largest entry with round_weights
+    // (operator form, M = 600 - 1000).
+    for (int m = 2; m <= N; ++m) {
+      double e[Q / 2] = {}, u[Q / 2] = {};
+      float r[Q / 2] = {};
+      for (int q = 0; q < Q / 2; ++q) {
+        u[q] = sd[q];
+        e[q] = gw[q % 3] / NQI * legendre_value(m, sd[q]);
+      }
+      round_weights<float, Q / 2>(e, u, m & 1, r);
+      for (int q = 0; q < Q / 2; ++q) {
+        W[m][q] = r[q];
+        W[m][Q - 1 - q] = (m & 1) ? -r[q] : r[q];
+      }
+    }
   }
 };
 
@@ -158,15 +204,10 @@ __host__ __device__ constexpr double gl_node(int NP, int h) {
 __host__ __device__ constexpr double gl_weight(int NP, int h) {
   return NP == 6 ? kGL6Weight[h] : (NP == 8 ? kGL8Weight[h] : kGL10Weight[h]);
 }
-// Rounding to FP32 must not leave a functional that is blind to constants
-// (even m >= 2) with a sum of its own: over thousands of sources of one sign
-// (the right-hand side's) that sum, 1e-8 of G_0 each, would add up.  So the
-// smallest weight of each mode absorbs the others' rounding: the even modes
-// then reproduce the functional of 1, the odd ones that of s.
-template <int N, int NP>
+template <int N, int NP, class Real = float>
 struct FarWeights {
   static constexpr int H = NP / 2;
-  float W[H][N + 1];
+  Real W[H][N + 1];
   constexpr FarWeights() : W() {}
   constexpr FarWeights(int NQI, bool exact) : W() {
     double x[NP] = {}, acc[H][N + 1] = {};
@@ -194,17 +235,14 @@ struct FarWeights {
         }
     }
     for (int m = 0; m <= N; ++m) {
-      int least = 0;
-      double sum = 0.0;  // the functional of 1 or s, less the rounded weights'
+      double e[H] = {}, u[H] = {};
+      Real r[H] = {};
       for (int h = 0; h < H; ++h) {
-        W[h][m] = static_cast<float>(acc[h][m]);
-        const double u = (m & 1) ? x[h] : 1.0;
-        sum += (acc[h][m] - static_cast<double>(W[h][m])) * u;
-        const double mag = acc[h][m] < 0.0 ? -acc[h][m] : acc[h][m];
-        const double low = acc[least][m] < 0.0 ? -acc[least][m] : acc[least][m];
-        if (mag < low) least = h;
+        e[h] = acc[h][m];
+        u[h] = x[h];
       }
-      W[least][m] = static_cast<float>(W[least][m] + sum / ((m & 1) ? x[least] : 1.0));
+      round_weights<Real, H>(e, u, m & 1, r);
+      for (int h = 0; h < H; ++h) W[h][m] = r[h];
     }
   }
 };

@@ -24,6 +24,11 @@ int max_pair_groups(int M);
 // orientations are [3*M] FP64 device arrays.
 hipError_t launch_assemble(int N, int NQI, bool analytical, int M, int64_t lda, const double* pos,
                            const double* ori, float* A, double* bpart, const PhysConsts& pc, hipStream_t s);
+// Dense columns of source fibers j0 .. j0 + jcount - 1 from the state (leading
+// dimension lda, source fiber j0's first column at A[0]); no right-hand side.
+hipError_t launch_assemble_columns(int N, int NQI, bool analytical, int M, int64_t lda, const double* pos,
+                                   const double* ori, float* A, const PhysConsts& pc, hipStream_t s, int j0,
+                                   int jcount);
 hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double* out, hipStream_t s);
 
 // Theta form (rf_assemble.hip): T holds NC = 3 + 6(N-1) component arrays of
@@ -33,6 +38,13 @@ hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double
 // (Theta_0 and Phi0 of every source mode) and the velocity constants
 // cpart[group][i][6] (cpart then holds max_pair_groups(M) * M * 6 doubles).
 PairGrid theta_grid(int M, int sources_per_iteration);
+// Below this many fibers every pair takes the near kernel alone: the launch is
+// then its latency, and the far kernel's own (24 us at M = 100: a few wavefronts
+// with one batch after another) is longer than what it takes off the near one's.
+// Assembly in us, near alone / with the far kernel, at 0.1 fibers per unit
+// volume: numerical M = 200 78 / 84, 250 107 / 95, 400 187 / 126; analytical
+// 300 103 / 124, 400 140 / 131, 600 243 / 196.
+__host__ __device__ constexpr int far_min_fibers(bool analytical) { return analytical ? 384 : 240; }
 // The far pairs (rf_far.hip): their sums go to the partial slots after the near
 // pairs' (slot0 on).
 PairGrid far_grid(int M);
@@ -49,6 +61,62 @@ hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t
 // rows sum_{j in group} A_ij x0_j into apart[group len + row].  With T16 it
 // also writes the FP16 copy of T with one FP32 scale per (target, source)
 // block, S16[i * M + j] = max |T_ij| / 32768 (the GMRES-IR inner system).
+// The system of a large suspension for the iterative solvers (rf_operator.hip):
+// the pairs of far_rule's first radius and beyond are not stored; a product
+// forms their kernel values again.  The others are, per target fiber, in the
+// theta form's components: `data` holds segments of floats, target i's at
+// base[i] (in floats) with its count[i] sources as ints, padded to 16, then NC
+// (and, with the velocity operator, 12 more) rows of near_stride(count, N)
+// floats, column slot N + k_j.
+struct NearStore {
+  float* data;
+  int64_t capacity;           // floats
+  unsigned long long* used;   // floats taken (device); more than capacity: the launch has to be repeated
+  int64_t* base;
+  int* count;
+  int velocity;               // the segments hold the velocity operator
+};
+__host__ __device__ inline int near_ints(int count) { return (count + 15) / 16 * 16; }
+__host__ __device__ inline int64_t near_stride(int count, int N) {
+  return (static_cast<int64_t>(count) * N + 15) / 16 * 16;
+}
+// Whether the iterative solvers take this form: from the size on where the
+// stored form (540 bytes per pair for N = 5) no longer stays in the caches and a
+// product is its HBM pass.  Step time in us, stored / operator: N = 5 at 0.03
+// fibers per unit volume (numerical) M = 700 916 / 892, 1000 1353 / 1043, 2000
+// 4289 / 2055, at 0.1 (analytical) 700 1136 / 1203, 1000 3234 / 2694, 2000 5710 /
+// 2896; N = 8 350 1200 / 1272, 500 1614 / 1405, 1000 3659 / 1824; N = 3 1000 842 /
+// 997, 1600 1566 / 1578, 2000 2174 / 2117.  N = 1 and 2 store at most 72 bytes per
+// pair, less than the kernel values cost.
+inline bool operator_form(int M, int N) {
+  const double stored = 4.0 * M * static_cast<double>(M) * N * (3 + 6 * (N - 1));
+  return N >= 3 && stored >= 450e6;
+}
+// Workspace of the products.
+struct Operator {
+  NearStore near;
+  double* nodes;  // op_node_doubles
+  double* part;   // op_part_doubles
+};
+size_t op_node_doubles(int M, int N);
+size_t op_part_doubles(int M, int N);
+// The near pairs' segments, and their sums as launch_assemble_theta writes
+// them, into slot 0 of bpart, cpart and apart.
+hipError_t launch_assemble_near(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
+                                const NearStore& near, double* bpart, double* cpart, const double* x0, double* apart,
+                                const PhysConsts& pc, hipStream_t s);
+// The far pairs' sums into slot 1.
+hipError_t op_assemble_far(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
+                           const Operator& op, double* bpart, double* cpart, const double* x0, double* apart,
+                           const PhysConsts& pc, hipStream_t s);
+// y = A x (mode 0) or y = b - A x (mode 1).
+hipError_t op_product(int N, int NQI, bool analytical, int M, const double* pos, const double* ori, const Operator& op,
+                      const double* x, double* y, const double* b, int mode, const PhysConsts& pc, hipStream_t s,
+                      hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr, const int* skip = nullptr);
+// Velocities from the solution x; cpart's two slots as the assembly wrote them.
+hipError_t op_velocities(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
+                         const Operator& op, const double* cpart, const double* x, const PhysConsts& pc, double* tvel,
+                         double* rvel, hipStream_t s);
 // r = b - (x0 + sum_g apart[g]): the residual of x0 from those partials.
 hipError_t launch_residual_groups(int groups, int64_t len, const double* apart, const double* b, const double* x0,
                                   double* r, hipStream_t s);
