@@ -51,7 +51,9 @@ typedef enum rf_solver {
   RF_SOLVER_DIRECT_MIXED_BF16 = 3, /* BF16-MFMA LU + FP64 iterative refinement */
   RF_SOLVER_DIRECT_MIXED_FP16 = 4, /* FP16-MFMA LU + FP64 iterative refinement */
   RF_SOLVER_GMRES_IR = 5           /* GMRES on the FP16-stored theta system inside an iterative refinement
-                                      whose residual uses the FP32 theta system in FP64 */
+                                      whose residual uses the FP32 theta system in FP64; large suspensions
+                                      under RF_MATRIX_AUTO, whose far pairs are not stored, take the same
+                                      products inside and outside */
 } rf_solver;
 
 /* --numerical / --analytical (fibers_runner.py:105-108). */
@@ -85,7 +87,11 @@ typedef enum rf_initial_guess {
  * as the 3 + 6(N-1) numbers that determine a block column (Q0 and the
  * symmetric projections Theta, fortran/assemble_matrix.incl:59-137), 40% fewer
  * bytes for N = 5; the matrix-vector product rebuilds the blocks on the fly.
- * AUTO: THETA.  The direct solvers expand the theta form into their factor
+ * AUTO: THETA, except that the iterative solvers of large suspensions (N >= 3
+ * and 4 M^2 N (3 + 6 (N - 1)) bytes of it >= 450 MB: from about 900 fibers for
+ * N = 5) store the pairs near each other only and form the others' kernel
+ * values in each product: the same system to FP32 rounding, without the HBM
+ * pass over it.  The direct solvers expand the theta form into their factor
  * storage and refine with the theta matrix-vector product; with DENSE they
  * copy the dense matrix and refine with the dense product.  Dumps
  * (rf_get_system) always return the dense matrix. */
@@ -162,7 +168,8 @@ typedef struct rf_timings {
   int32_t gemm_launches;   /* direct solvers: trailing-update GEMMs of the LU factorisation (built-in MFMA kernel) */
   double gemm;             /* their summed duration */
   double gemm_flop;        /* their algorithmic flops, 2 m n K each */
-  double gemv_half;        /* GMRES-IR: summed duration of the FP16 matrix-vector kernels */
+  double gemv_half;        /* GMRES-IR: summed duration of the FP16 matrix-vector kernels (none on the operator
+                              form) */
   int32_t gemv_half_launches;
   int32_t direct_fallback; /* direct solvers: 1 when the refinement did not converge and GMRES on the dense
                               system finished the solve (iterations then count both) */
