@@ -270,7 +270,6 @@ struct CycleHead {
   int k_used;     // its Arnoldi steps
   int nonfinite;  // a non-finite ||w|| ended it
   int pad;
-  double scale;   // 1 / ||w|| of the last step: normalises V_{k+1}
   double res;     // |g_k|, the cycle's residual estimate
 };
 struct CycleCtl {
@@ -285,7 +284,7 @@ struct CycleCtl {
 // Device doubles of a cycle's control (head included), and its layout in them.
 size_t cycle_ctl_doubles(int m);
 CycleCtl cycle_ctl(double* mem, int m);
-// Dot partials of the steps: 3 (m + 1) mdot_blocks(n) doubles.
+// Dot partials of the steps.
 size_t cycle_part_doubles(int64_t n, int m);
 // g = (beta, 0, ..., 0), head cleared.
 hipError_t cycle_start(const CycleCtl& c, int m, double beta, hipStream_t s);

@@ -817,12 +817,17 @@ hipError_t gemv_theta16(int N, int M, int64_t Lp, const _Float16* T16, const flo
 // ---------------------------------------------------------------------------
 // Single-simulation GMRES(m), a restart cycle with its control on the
 // device (the reference's solver reads and writes the Hessenberg entries on
-// the host at every step, lib/viennacl/linalg/gmres.hpp:246,281-285).  A
-// step is 7 launches after its product: the dots and the update of each
-// Gram-Schmidt pass (the update forms the coefficients from the dots' block
-// partials itself), ||w||^2, the control step and the normalisation.  Each
-// coefficient is the sum of its block partials in block order, the same in
-// the update and in the control.
+// the host at every step, lib/viennacl/linalg/gmres.hpp:246,281-285).
+//
+// What a step costs beside its product is launches (about 5 us each in a chain)
+// more than work.  Short vectors (kOneGroupRows, kOneGroupWork): one workgroup
+// does the whole step, the vector in registers, in one launch: 7 - 17 us at
+// n = 1 500 (K = 1 - 5) against 43 us for seven launches, a step of the solver 51
+// instead of 68 us.  Else four launches: the dots of the
+// first Gram-Schmidt pass, its update with the dots of the second on the same
+// rows, that update with ||w||^2, and the control step with the normalisation.
+// A coefficient is the sum of its block partials in one order wherever it is
+// formed.
 
 size_t cycle_ctl_doubles(int m) {
   return sizeof(CycleHead) / sizeof(double) + static_cast<size_t>(m + 1) * m + 4 * static_cast<size_t>(m) + 1;
@@ -841,13 +846,16 @@ CycleCtl cycle_ctl(double* mem, int m) {
   return c;
 }
 
-size_t cycle_part_doubles(int64_t n, int m) { return 3 * static_cast<size_t>(m + 1) * mdot_blocks(n); }
-
-__device__ __forceinline__ double sum_parts(const double* __restrict__ p, int nb) {
-  double s = 0.0;
-  for (int b = 0; b < nb; ++b) s += p[b];
-  return s;
+// Rows of a workgroup in the vector passes: few enough that the launch has some
+// hundred workgroups, as many as leave them no more than that many partials to
+// sum.  Solve of 8 steps at n = 14 424: 1024 rows 2.012 ms, 512 1.977, 256 1.964;
+// at 30 000 1.431, 1.399, 1.390; at 75 000 6.068, 6.037, 6.077.
+static int64_t pass_rows(int64_t n) {
+  return n <= 48 * 1024 ? 256 : (n <= 128 * 1024 ? 512 : (n <= 256 * 1024 ? 1024 : 4096));
 }
+static int pass_blocks(int64_t n) { return static_cast<int>((n + pass_rows(n) - 1) / pass_rows(n)); }
+
+size_t cycle_part_doubles(int64_t n, int m) { return 3 * static_cast<size_t>(m + 1) * pass_blocks(n); }
 
 __global__ void cycle_start_kernel(CycleCtl c, int m, double beta) {
   for (int i = threadIdx.x; i <= m; i += blockDim.x) c.g[i] = (i == 0) ? beta : 0.0;
@@ -856,44 +864,93 @@ __global__ void cycle_start_kernel(CycleCtl c, int m, double beta) {
     c.head->k_used = 0;
     c.head->nonfinite = 0;
     c.head->pad = 0;
-    c.head->scale = 1.0;
     c.head->res = beta;
     if (c.hdone) *c.hdone = 0;
   }
 }
 
-// w -= sum_{k < K} V_k h_k with h_k the sum of the dots' block partials of V_k.
-__global__ __launch_bounds__(256) void cgs_update_kernel(int64_t n, int K, const double* __restrict__ V, int64_t ldv,
-                                                         const double* __restrict__ part, int nb,
-                                                         double* __restrict__ w, const int* __restrict__ skip) {
-  extern __shared__ double h[];
-  if (*skip) return;
-  for (int k = threadIdx.x; k < K; k += blockDim.x) h[k] = sum_parts(part + static_cast<int64_t>(k) * nb, nb);
-  __syncthreads();
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (r >= n) return;
+// Sum of one reduction's block partials by the lanes of a wavefront (every lane
+// returns it).
+__device__ __forceinline__ double wave_sum(const double* __restrict__ p, int nb) {
   double s = 0.0;
-  for (int k = 0; k < K; ++k) s = fma(V[static_cast<int64_t>(k) * ldv + r], h[k], s);
-  w[r] = fma(-1.0, s, w[r]);
+  for (int b = threadIdx.x & 63; b < nb; b += 64) s += p[b];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  return s;
 }
 
-// The control of step k: H(:, k) = h0 + h1 and ||w||, the earlier rotations
-// and a new one, g and the estimate |g_{k+1}|; at the cycle's end y = H^-1 g.
-__global__ __launch_bounds__(64) void arnoldi_step_kernel(int k, int klast, int m, int nb,
-                                                          const double* __restrict__ part, double tol, double bnorm,
-                                                          CycleCtl c) {
-  extern __shared__ double hs[];  // h0[K], h1[K], ||w||^2
-  CycleHead& hd = *c.head;
-  if (hd.done) return;
-  const int K = k + 1;
-  const int64_t region = static_cast<int64_t>(m + 1) * nb;
-  for (int t = threadIdx.x; t <= 2 * K; t += blockDim.x) {
-    const int p = t < K ? 0 : (t < 2 * K ? 1 : 2);
-    const int j = t < K ? t : (t < 2 * K ? t - K : 0);
-    hs[t] = sum_parts(part + p * region + static_cast<int64_t>(j) * nb, nb);
+// One vector pass on the workgroup's rows of w: after the first (phase 0),
+// w -= sum_{k < K} V_k h_k with h_k from the last phase's partials; then the
+// partials of <V_k, w>, k < K (phases 0 and 1), or of ||w||^2 (phase 2).
+constexpr int kPassChunk = 8;  // dots reduced at a time
+__global__ __launch_bounds__(256) void arnoldi_pass_kernel(int64_t n, int64_t rows, int phase, int K, int64_t region,
+                                                           const double* __restrict__ V, double* __restrict__ w,
+                                                           double* __restrict__ part, const int* __restrict__ skip) {
+  extern __shared__ double sh[];  // w of the rows, then h[K], then the wavefronts' partials
+  if (*skip) return;
+  double* const ws = sh;
+  double* const h = sh + rows;
+  double* const red = h + K;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nb = gridDim.x;
+  const int64_t lo = static_cast<int64_t>(blockIdx.x) * rows;
+  const int cnt = static_cast<int>(min(rows, n - lo));
+  if (phase > 0) {
+    for (int k = wave; k < K; k += 4) {
+      const double v = wave_sum(part + (phase - 1) * region + static_cast<int64_t>(k) * nb, nb);
+      if (lane == 0) h[k] = v;
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
+  for (int r = threadIdx.x; r < cnt; r += 256) {
+    double v = w[lo + r];
+    if (phase > 0) {
+      double s = 0.0;
+      for (int k = 0; k < K; ++k) s = fma(V[static_cast<int64_t>(k) * n + lo + r], h[k], s);
+      v = fma(-1.0, s, v);
+      w[lo + r] = v;
+    }
+    ws[r] = v;
+  }
+  // a lane reads back only the rows it wrote
+  const int J = phase == 2 ? 1 : K;
+  for (int k0 = 0; k0 < J; k0 += kPassChunk) {
+    double d[kPassChunk];
+#pragma unroll
+    for (int q = 0; q < kPassChunk; ++q) d[q] = 0.0;
+    for (int r = threadIdx.x; r < cnt; r += 256) {
+      const double v = ws[r];
+      if (phase == 2) {
+        d[0] = fma(v, v, d[0]);
+      } else {
+#pragma unroll
+        for (int q = 0; q < kPassChunk; ++q)
+          if (k0 + q < K) d[q] = fma(V[static_cast<int64_t>(k0 + q) * n + lo + r], v, d[q]);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kPassChunk; ++q) {
+      if (k0 + q >= J) break;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) d[q] += __shfl_xor(d[q], off, 64);
+      if (lane == 0) red[wave * kPassChunk + q] = d[q];
+    }
+    __syncthreads();
+    if (threadIdx.x < kPassChunk && k0 + static_cast<int>(threadIdx.x) < J) {
+      double t = 0.0;
+      for (int q = 0; q < 4; ++q) t += red[q * kPassChunk + threadIdx.x];
+      part[phase * region + static_cast<int64_t>(k0 + threadIdx.x) * nb + blockIdx.x] = t;
+    }
+    __syncthreads();
+  }
+}
+
+// The control of step k, by one lane: H(:, k) = h0 + h1 and ||w||, the earlier
+// rotations and a new one, g and the estimate |g_{k+1}|; at the cycle's end
+// y = H^-1 g.  hs: h0[K], h1[K], ||w||^2.
+__device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const double* hs, double tol, double bnorm,
+                                                const CycleCtl& c) {
+  CycleHead& hd = *c.head;
+  const int K = k + 1;
   const double hn = sqrt(hs[2 * K]);
   if (!isfinite(hn)) {
     hd.nonfinite = 1;
@@ -929,15 +986,114 @@ __global__ __launch_bounds__(64) void arnoldi_step_kernel(int k, int klast, int 
     hd.k_used = K;
     hd.done = 1;
     if (c.hdone) *c.hdone = 1;
-  } else {
-    hd.scale = 1.0 / hn;
   }
 }
 
-__global__ void arnoldi_scale_kernel(int64_t n, double* __restrict__ w, const CycleHead* __restrict__ hd) {
-  if (hd->done) return;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (r < n) w[r] = hd->scale * w[r];
+// w /= ||w|| in every workgroup, the control in the first (a workgroup that
+// starts after it ended the cycle returns: the vector is not read any more).
+__global__ __launch_bounds__(256) void arnoldi_finish_kernel(int64_t n, int nb, int k, int klast, int m,
+                                                             int64_t region, const double* __restrict__ part,
+                                                             double* __restrict__ w, double tol, double bnorm,
+                                                             CycleCtl c) {
+  extern __shared__ double hs[];  // first workgroup: h0[K], h1[K], ||w||^2
+  if (c.head->done) return;
+  const int K = k + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double hn = sqrt(wave_sum(part + 2 * region, nb));
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (r < n && isfinite(hn) && hn > 0.0) w[r] = (1.0 / hn) * w[r];
+  if (blockIdx.x != 0) return;
+  for (int t = wave; t <= 2 * K; t += 4) {
+    const int p = t < K ? 0 : (t < 2 * K ? 1 : 2);
+    const int j = t < K ? t : (t < 2 * K ? t - K : 0);
+    const double v = wave_sum(part + p * region + static_cast<int64_t>(j) * nb, nb);
+    if (lane == 0) hs[t] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) arnoldi_control(k, klast, m, hs, tol, bnorm, c);
+}
+
+// The whole step in one workgroup: w in registers, each Gram-Schmidt pass's
+// dots kPassChunk at a time.
+constexpr int kOneGroup = 1024;
+constexpr int kOneGroupRows = 8192;   // 8 per lane
+constexpr int kOneGroupWork = 65536;  // n K: beyond it one CU's loads of V take longer than the launches
+__global__ __launch_bounds__(kOneGroup) void arnoldi_one_kernel(int n, int k, int klast, int m,
+                                                                const double* __restrict__ V, double* __restrict__ w,
+                                                                double tol, double bnorm, CycleCtl c) {
+  constexpr int R = kOneGroupRows / kOneGroup, W = kOneGroup / 64;
+  extern __shared__ double hs[];  // h0[K], h1[K], ||w||^2
+  __shared__ double red[W][kPassChunk];
+  if (c.head->done) return;
+  const int K = k + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int R0 = (n + kOneGroup - 1) / kOneGroup;
+  double wr[R];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int r = static_cast<int>(threadIdx.x) + q * kOneGroup;
+    wr[q] = r < n ? w[r] : 0.0;
+  }
+  auto reduce = [&](double (&d)[kPassChunk], int cnt, double* out) {
+#pragma unroll
+    for (int q = 0; q < kPassChunk; ++q) {
+      if (q >= cnt) break;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) d[q] += __shfl_xor(d[q], off, 64);
+      if (lane == 0) red[wave][q] = d[q];
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < cnt) {
+      double t = 0.0;
+#pragma unroll
+      for (int q = 0; q < W; ++q) t += red[q][threadIdx.x];
+      out[threadIdx.x] = t;
+    }
+    __syncthreads();
+  };
+  for (int pass = 0; pass < 2; ++pass) {
+    double* const h = hs + pass * K;
+    for (int k0 = 0; k0 < K; k0 += kPassChunk) {
+      double d[kPassChunk];
+#pragma unroll
+      for (int q = 0; q < kPassChunk; ++q) {
+        d[q] = 0.0;
+        if (k0 + q < K) {
+          const double* v = V + static_cast<int64_t>(k0 + q) * n;
+#pragma unroll
+          for (int e = 0; e < R; ++e) {
+            const int r = static_cast<int>(threadIdx.x) + e * kOneGroup;
+            if (e < R0 && r < n) d[q] = fma(v[r], wr[e], d[q]);
+          }
+        }
+      }
+      reduce(d, min(kPassChunk, K - k0), h + k0);
+    }
+    double s[R];
+#pragma unroll
+    for (int e = 0; e < R; ++e) s[e] = 0.0;
+    for (int j = 0; j < K; ++j) {
+      const double* v = V + static_cast<int64_t>(j) * n;
+      const double hj = h[j];
+#pragma unroll
+      for (int e = 0; e < R; ++e) {
+        const int r = static_cast<int>(threadIdx.x) + e * kOneGroup;
+        if (e < R0 && r < n) s[e] = fma(v[r], hj, s[e]);
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < R; ++e) wr[e] = fma(-1.0, s[e], wr[e]);
+  }
+  double d[kPassChunk] = {};
+#pragma unroll
+  for (int e = 0; e < R; ++e) d[0] = fma(wr[e], wr[e], d[0]);
+  reduce(d, 1, hs + 2 * K);
+  const double hn = sqrt(hs[2 * K]);
+  const double scale = isfinite(hn) && hn > 0.0 ? 1.0 / hn : 1.0;
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int r = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    if (r < n) w[r] = scale * wr[e];
+  }
+  if (threadIdx.x == 0) arnoldi_control(k, klast, m, hs, tol, bnorm, c);
 }
 
 __global__ void cycle_update_kernel(int64_t n, const double* __restrict__ V, CycleCtl c, double* __restrict__ x) {
@@ -958,22 +1114,23 @@ hipError_t cycle_start(const CycleCtl& c, int m, double beta, hipStream_t s) {
 hipError_t arnoldi_step(int64_t n, int k, int klast, int m, const double* V, double* w, double* part, double tol,
                         double bnorm, const CycleCtl& c, hipStream_t s) {
   if (k < 0 || k > klast || klast >= m) return hipErrorInvalidValue;
-  const int nb = mdot_blocks(n);
-  const int64_t rpb = (n + nb - 1) / nb;
-  const int64_t region = static_cast<int64_t>(m + 1) * nb;
   const int K = k + 1;
-  const unsigned vb = static_cast<unsigned>((n + 255) / 256);
-  const int* skip = &c.head->done;  // address arithmetic only
-  for (int pass = 0; pass < 2; ++pass) {
-    double* pp = part + pass * region;
-    hipLaunchKernelGGL(mdot_partial_kernel, dim3(nb, K), dim3(kDotThreads), 0, s, n, rpb, V, n, w, pp, skip);
-    hipLaunchKernelGGL(cgs_update_kernel, dim3(vb), dim3(256), K * sizeof(double), s, n, K, V, n, pp, nb, w, skip);
+  const size_t hbytes = (2 * static_cast<size_t>(K) + 1) * sizeof(double);
+  if (n <= kOneGroupRows && n * K <= kOneGroupWork) {
+    hipLaunchKernelGGL(arnoldi_one_kernel, dim3(1), dim3(kOneGroup), hbytes, s, static_cast<int>(n), k, klast, m, V, w,
+                       tol, bnorm, c);
+    return hipGetLastError();
   }
-  hipLaunchKernelGGL(mdot_partial_kernel, dim3(nb, 1), dim3(kDotThreads), 0, s, n, rpb, w, n, w, part + 2 * region,
-                     skip);
-  hipLaunchKernelGGL(arnoldi_step_kernel, dim3(1), dim3(64), (2 * K + 1) * sizeof(double), s, k, klast, m, nb, part,
-                     tol, bnorm, c);
-  hipLaunchKernelGGL(arnoldi_scale_kernel, dim3(vb), dim3(256), 0, s, n, w, c.head);
+  const int64_t rows = pass_rows(n);
+  const int nb = pass_blocks(n);
+  const int64_t region = static_cast<int64_t>(m + 1) * nb;
+  const int* skip = &c.head->done;  // address arithmetic only
+  const size_t pbytes = (static_cast<size_t>(rows) + K + 4 * kPassChunk) * sizeof(double);
+  for (int phase = 0; phase < 3; ++phase)
+    hipLaunchKernelGGL(arnoldi_pass_kernel, dim3(nb), dim3(256), pbytes, s, n, rows, phase, K, region, V, w, part,
+                       skip);
+  hipLaunchKernelGGL(arnoldi_finish_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), hbytes, s, n, nb,
+                     k, klast, m, region, static_cast<const double*>(part), w, tol, bnorm, c);
   return hipGetLastError();
 }
 
@@ -986,7 +1143,9 @@ hipError_t cycle_update(int64_t n, const double* V, const CycleCtl& c, double* x
 // BiCGStab with its scalars on the device.  Each scalar kernel is one wave
 // that sums the dots' block partials exactly as mdot_final_kernel does, and
 // each vector kernel repeats the axpby sequence of the host form, so the
-// iterates are the ones host-side scalars give.
+// iterates are the ones host-side scalars give.  Vectors of at most
+// kOneGroupRows: one workgroup does what follows each product, in one launch
+// instead of six.
 
 size_t bicg_part_doubles(int64_t n) { return 6 * static_cast<size_t>(mdot_blocks(n)); }
 
@@ -1171,7 +1330,184 @@ hipError_t bicg_start(const BicgCtl& c, double rho, double res, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Sums over the workgroup of kOneGroup lanes, every lane returning them.
+template <int S>
+__device__ __forceinline__ void one_group_sums(double (&d)[S], double (*red)[2]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) d[q] += __shfl_xor(d[q], off, 64);
+    if (lane == 0) red[wave][q] = d[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+    d[q] = 0.0;
+#pragma unroll
+    for (int v = 0; v < kOneGroup / 64; ++v) d[q] += red[v][q];
+  }
+  __syncthreads();
+}
+
+// What follows v = A p (bicg_alpha, _s, _snorm, _early) in one workgroup.
+__global__ __launch_bounds__(kOneGroup) void bicg_v_one_kernel(int n, int it, BicgVecs w, double tol, double bnorm,
+                                                               BicgCtl c) {
+  constexpr int R = kOneGroupRows / kOneGroup;
+  __shared__ double red[kOneGroup / 64][2];
+  BicgHead& h = *c.head;
+  if (h.done) return;
+  const double rho = h.rho;
+  const double* r0 = w.r + n;
+  double v[R], r[R], d[1] = {0.0};
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    v[e] = i < n ? w.v[i] : 0.0;
+    r[e] = i < n ? w.r[i] : 0.0;
+    if (i < n) d[0] = fma(r0[i], v[e], d[0]);
+  }
+  one_group_sums<1>(d, red);
+  const double r0v = d[0];
+  if (threadIdx.x == 0) {
+    ++h.its;
+    ++h.prods;
+  }
+  if (r0v == 0.0 || !isfinite(r0v)) {
+    if (threadIdx.x == 0) bicg_end(c);
+    return;
+  }
+  const double alpha = rho / r0v;
+  d[0] = 0.0;
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    const double si = fma(-alpha, v[e], 1.0 * r[e]);
+    if (i < n) {
+      w.s[i] = si;
+      d[0] = fma(si, si, d[0]);
+    }
+  }
+  one_group_sums<1>(d, red);
+  const double snorm = sqrt(d[0]);
+  const bool bad = !isfinite(snorm), early = !bad && snorm / bnorm <= tol;
+  if (threadIdx.x == 0) {
+    h.alpha = alpha;
+    if (bad) {
+      h.nonfinite = 1;
+      bicg_end(c);
+    } else if (early) {
+      h.res = snorm;
+      h.converged = 1;
+      h.early_it = it;
+      bicg_end(c);
+    }
+  }
+  if (!early) return;
+  for (int i = threadIdx.x; i < n; i += kOneGroup) w.x[i] = fma(alpha, w.p[i], 1.0 * w.x[i]);
+}
+
+// What follows t = A s (bicg_omega, _xr, _end, _p) in one workgroup.
+__global__ __launch_bounds__(kOneGroup) void bicg_t_one_kernel(int n, BicgVecs w, double tol, double bnorm,
+                                                               BicgCtl c) {
+  constexpr int R = kOneGroupRows / kOneGroup;
+  __shared__ double red[kOneGroup / 64][2];
+  BicgHead& h = *c.head;
+  if (h.done) return;
+  const double alpha = h.alpha, rho = h.rho;
+  const int since = h.its - 1 - h.last_restart;
+  const double* r0 = w.r + n;
+  const double* t = w.s + n;
+  double sv[R], tv[R], d[2] = {0.0, 0.0};
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    sv[e] = i < n ? w.s[i] : 0.0;
+    tv[e] = i < n ? t[i] : 0.0;
+    d[0] = fma(sv[e], tv[e], d[0]);
+    d[1] = fma(tv[e], tv[e], d[1]);
+  }
+  one_group_sums<2>(d, red);
+  const double omega = (d[1] == 0.0) ? 0.0 : d[0] / d[1];
+  double r[R];
+  d[0] = d[1] = 0.0;
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    r[e] = fma(-omega, tv[e], 1.0 * (1.0 * sv[e]));
+    if (i < n) {
+      const double xi = fma(alpha, w.p[i], 1.0 * w.x[i]);
+      w.x[i] = fma(omega, sv[e], 1.0 * xi);
+      w.r[i] = r[e];
+      d[0] = fma(r[e], r[e], d[0]);
+      d[1] = fma(r0[i], r[e], d[1]);
+    }
+  }
+  one_group_sums<2>(d, red);
+  const double res = sqrt(d[0]), rho_new = d[1];
+  const bool bad = !isfinite(res), met = !bad && res / bnorm <= tol;
+  const bool restart = !bad && !met && (rho_new == 0.0 || omega == 0.0 || since > kBicgRestartEvery);
+  const double beta = (rho_new / rho) * (alpha / omega);
+  if (threadIdx.x == 0) {
+    ++h.prods;
+    h.omega = omega;
+    h.res = res;
+    if (bad) {
+      h.nonfinite = 1;
+      bicg_end(c);
+    } else if (met) {
+      h.converged = 1;
+      bicg_end(c);
+    } else if (restart) {
+      h.restart = 1;
+      h.no_restart = 0;
+    } else {
+      h.beta = beta;
+      h.rho = rho_new;
+    }
+  }
+  if (bad || met || restart) return;
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    if (i < n) {
+      const double q = fma(-omega, w.v[i], 1.0 * w.p[i]);
+      w.p[i] = fma(1.0, r[e], beta * q);
+    }
+  }
+}
+
+// A pending restart (bicg_restart_copy, _restart) in one workgroup.
+__global__ __launch_bounds__(kOneGroup) void bicg_restart_one_kernel(int n, BicgVecs w, BicgCtl c) {
+  __shared__ double red[kOneGroup / 64][2];
+  BicgHead& h = *c.head;
+  if (h.no_restart) return;
+  double d[1] = {0.0};
+  for (int i = threadIdx.x; i < n; i += kOneGroup) {
+    const double ri = w.r[i];
+    w.r[n + i] = ri;
+    w.p[i] = ri;
+    d[0] = fma(ri, ri, d[0]);
+  }
+  one_group_sums<1>(d, red);
+  if (threadIdx.x != 0) return;
+  h.rho = d[0];
+  h.res = sqrt(d[0]);
+  h.restart = 0;
+  h.no_restart = 1;
+  h.last_restart = h.its;
+  ++h.restarts;
+  if (!isfinite(d[0])) {
+    h.nonfinite = 1;
+    bicg_end(c);
+  }
+}
+
 hipError_t bicg_restart(int64_t n, const BicgVecs& w, double* part, const BicgCtl& c, hipStream_t s) {
+  if (n <= kOneGroupRows) {
+    hipLaunchKernelGGL(bicg_restart_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), w, c);
+    return hipGetLastError();
+  }
   const int nb = mdot_blocks(n);
   const int64_t rpb = (n + nb - 1) / nb;
   const unsigned vb = static_cast<unsigned>((n + 255) / 256);
@@ -1184,6 +1520,10 @@ hipError_t bicg_restart(int64_t n, const BicgVecs& w, double* part, const BicgCt
 
 hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, double tol, double bnorm,
                         const BicgCtl& c, hipStream_t s) {
+  if (n <= kOneGroupRows) {
+    hipLaunchKernelGGL(bicg_v_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), it, w, tol, bnorm, c);
+    return hipGetLastError();
+  }
   const int nb = mdot_blocks(n);
   const int64_t rpb = (n + nb - 1) / nb;
   const unsigned vb = static_cast<unsigned>((n + 255) / 256);
@@ -1202,6 +1542,10 @@ hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, doub
 
 hipError_t bicg_after_t(int64_t n, const BicgVecs& w, double* part, double tol, double bnorm, const BicgCtl& c,
                         hipStream_t s) {
+  if (n <= kOneGroupRows) {
+    hipLaunchKernelGGL(bicg_t_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), w, tol, bnorm, c);
+    return hipGetLastError();
+  }
   const int nb = mdot_blocks(n);
   const int64_t rpb = (n + nb - 1) / nb;
   const unsigned vb = static_cast<unsigned>((n + 255) / 256);
