@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -120,11 +121,13 @@ struct rf_simulation {
   double* gpart = nullptr;
   double* dpart = nullptr;
   double* hdev = nullptr;
-  int* flag = nullptr;
   rf::CycleCtl cyc{};  // GMRES: the device control of a restart cycle
   rf::BicgCtl bicg{};  // BiCGStab: its scalars on the device
-  int* hdone = nullptr;  // the done flag of either, mirrored into pinned host memory
-  hipEvent_t cev[2] = {nullptr, nullptr};  // the ends of the last two steps
+  // pinned host memory the device writes: the solve's mirror, and whether the
+  // velocities have a non-finite value
+  rf::SolveMirror* mirror = nullptr;
+  int* nonfinite = nullptr;
+  int* nonfinite_dev = nullptr;
   rf::GemvPlan plan{};
   rf::LuWorkspace lu{};
   rf::LuResult lu_last{};  // factorisation statistics of the last direct solve
@@ -270,14 +273,30 @@ hipError_t sim_gemv(rf_simulation* s, const double* x, double* part, double* y, 
   return rf::gemv(s->plan, s->A, x, part, y, b, mode, s->stream, e0, e1, skip);
 }
 
-rf_status check_nonfinite(rf_simulation* s, const double* v, int64_t len, const char* what) {
-  RF_HIP(hipMemsetAsync(s->flag, 0, sizeof(int), s->stream));
-  RF_HIP(rf::nonfinite_count(len, v, s->flag, s->stream));
-  int h = 0;
-  RF_HIP(hipMemcpyAsync(&h, s->flag, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-  RF_HIP(hipStreamSynchronize(s->stream));
-  if (h) return fail(RF_ERR_NONFINITE, std::string("non-finite values in ") + what);
-  return RF_OK;
+// Waits until the device control of the solve has run `steps` steps of the
+// cycle (or iterations) or ended it, by reading the pinned memory it writes: an
+// event's wait costs the host 35-45 us each time, more than a whole Krylov step
+// of a small system.  The stream's own state bounds the wait.
+rf_status wait_progress(rf_simulation* s, int steps) {
+  const volatile rf::SolveMirror* m = s->mirror;
+  for (unsigned spin = 1;; ++spin) {
+    if (m->done || m->progress >= steps) return RF_OK;
+    if (spin % 65536 != 0) {  // about 1 ms
+      __builtin_ia32_pause();
+      continue;
+    }
+    const hipError_t e = hipStreamQuery(s->stream);
+    if (e == hipErrorNotReady) continue;
+    if (e != hipSuccess) return fail(RF_ERR_DEVICE, std::string("solver: ") + hipGetErrorString(e));
+    // everything enqueued has run
+    if (m->done || m->progress >= steps) return RF_OK;
+    return fail(RF_ERR_DEVICE, "the solver's control did not report its progress");
+  }
+}
+
+void reset_mirror(rf_simulation* s) {
+  std::memset(static_cast<void*>(s->mirror), 0, sizeof(*s->mirror));
+  std::atomic_thread_fence(std::memory_order_seq_cst);
 }
 
 // ||v||_2 on the device, returned to the host (synchronises).
@@ -310,69 +329,64 @@ rf_status gmres_core(rf_simulation* s, const double* b, double* x, bool warm, do
   double* V = s->V;
   auto Vk = [&](int k) { return V + static_cast<int64_t>(k) * n; };
 
-  double bnorm = 0.0;
-  RF_TRY(device_norm(s, b, &bnorm));
   if (!warm) RF_HIP(rf::fill(n, 0.0, x, s->stream));
   *out = rf_solver_stats{0, 0, 0.0};
-  if (!std::isfinite(bnorm)) return fail(RF_ERR_NONFINITE, "non-finite right-hand side");
-  if (bnorm == 0.0) {
-    RF_HIP(rf::fill(n, 0.0, x, s->stream));
-    out->converged = 1;
-    return RF_OK;
-  }
   int it = 0;
   bool first = true, converged = false;
-  double res = bnorm;
+  double res = 0.0, bnorm = 0.0;
+  const volatile rf::SolveMirror* mir = s->mirror;
   while (true) {
-    double beta;
-    if (first && !warm) {
-      RF_HIP(rf::axpby(n, 1.0, b, 0.0, Vk(0), s->stream));
-      beta = bnorm;
-      first = false;
-    } else if (first && r0) {
-      first = false;
-      RF_HIP(rf::axpby(n, 1.0, r0, 0.0, Vk(0), s->stream));
-      RF_TRY(device_norm(s, Vk(0), &beta));
-    } else {
-      first = false;
+    const double* r = Vk(0);
+    if (first && !warm)
+      r = b;
+    else if (first && r0)
+      r = r0;
+    else
       RF_HIP(sim_gemv(s, x, s->gpart, Vk(0), b, 1, half));
-      RF_TRY(device_norm(s, Vk(0), &beta));
-    }
-    res = beta;
-    if (!std::isfinite(beta)) return fail(RF_ERR_NONFINITE, "non-finite residual in GMRES");
-    if (beta / bnorm <= tol) {
-      converged = true;
-      break;
-    }
-    if (it >= maxit) break;
-    RF_HIP(rf::axpby(n, 1.0 / beta, Vk(0), 0.0, Vk(0), s->stream));
-    // The control of the cycle runs on the device; the host stays one step
-    // ahead: it enqueues step k + 1, then waits for the end of step k and
-    // reads the done flag that step's control mirrors into host memory.  The
-    // product and vector kernels of a step enqueued after the cycle's end
-    // return at once (at most one per cycle).
+    first = false;
+    // The control of the cycle, its start included, runs on the device; the
+    // host stays one step ahead: it enqueues step k + 1, then waits for the
+    // control of step k, which it sees in pinned memory.  The product and
+    // vector kernels of a step enqueued after the cycle's end return at once
+    // (at most one per cycle).
     const int steps = std::min(m, maxit - it);
     int& launched = half && !s->oper ? s->nhalf : s->ngemv;
     const int launched0 = launched;
-    RF_HIP(rf::cycle_start(s->cyc, m, beta, s->stream));
+    reset_mirror(s);
+    RF_HIP(rf::cycle_start(n, s->cyc, m, b, r, Vk(0), s->dpart, tol, s->stream));
     for (int k = 0; k < steps; ++k) {
       RF_HIP(sim_gemv(s, Vk(k), s->gpart, Vk(k + 1), nullptr, 0, half, &s->cyc.head->done));
-      RF_HIP(rf::arnoldi_step(n, k, steps - 1, m, V, Vk(k + 1), s->dpart, tol, bnorm, s->cyc, s->stream));
-      RF_HIP(hipEventRecord(s->cev[k & 1], s->stream));
+      RF_HIP(rf::arnoldi_step(n, k, steps - 1, m, V, Vk(k + 1), s->dpart, tol, s->cyc, s->stream));
       if (k > 0) {
-        RF_HIP(hipEventSynchronize(s->cev[(k - 1) & 1]));
-        if (*static_cast<volatile int*>(s->hdone)) break;
+        RF_TRY(wait_progress(s, k));
+        if (mir->done) break;
       }
     }
-    RF_HIP(rf::cycle_update(n, V, s->cyc, x, s->stream));
-    rf::CycleHead hd{};
-    RF_HIP(hipMemcpyAsync(&hd, s->cyc.head, sizeof(hd), hipMemcpyDeviceToHost, s->stream));
-    RF_HIP(hipStreamSynchronize(s->stream));
+    if (steps > 0) {
+      RF_HIP(rf::cycle_update(n, V, s->cyc, x, s->stream));
+      RF_TRY(wait_progress(s, m + 1));  // its last step ends a cycle
+    } else {
+      RF_HIP(hipStreamSynchronize(s->stream));
+    }
     // products that returned at once are not counted (nor timed)
-    launched = std::min(launched, launched0 + hd.k_used + hd.nonfinite);
-    it += hd.k_used + hd.nonfinite;
-    if (hd.nonfinite) return fail(RF_ERR_NONFINITE, "non-finite Arnoldi vector in GMRES");
-    res = hd.res;
+    const int used = mir->used, nonfinite = mir->nonfinite, start = mir->start;
+    launched = std::min(launched, launched0 + used + (nonfinite == 1));
+    res = mir->res;
+    bnorm = mir->bnorm;
+    if (nonfinite == 2) return fail(RF_ERR_NONFINITE, "non-finite right-hand side");
+    if (nonfinite == 3) return fail(RF_ERR_NONFINITE, "non-finite residual in GMRES");
+    if (nonfinite) return fail(RF_ERR_NONFINITE, "non-finite Arnoldi vector in GMRES");
+    if (start == 1) {  // b = 0
+      RF_HIP(rf::fill(n, 0.0, x, s->stream));
+      out->converged = 1;
+      return RF_OK;
+    }
+    if (start == 2) {
+      converged = true;
+      break;
+    }
+    if (steps <= 0) break;
+    it += used;
     if (!confirm && res / bnorm <= tol) {
       converged = true;
       break;
@@ -485,82 +499,83 @@ rf_status solve_bicgstab(rf_simulation* s) {
   s->bicg_restarts = 0;
   const int maxit = s->cfg.bicgstab_max_iterations;
   const double tol = s->cfg.bicgstab_tolerance;
-  double* r = s->work;
-  double* r0 = s->work + n;
+  double* r = s->work;  // r0 follows it
   double* p = s->work + 2 * n;
   double* v = s->work + 3 * n;
   double* sv = s->work + 4 * n;
   double* t = s->work + 5 * n;
-  double bnorm = 0.0;
-  RF_TRY(device_norm(s, s->b, &bnorm));
   bool warm = false;
   const double* r0x = nullptr;
   RF_TRY(take_guess(s, &warm, &r0x));
   s->stats = rf_solver_stats{0, 0, 0.0};
-  if (!std::isfinite(bnorm)) return fail(RF_ERR_NONFINITE, "non-finite right-hand side");
-  if (bnorm == 0.0 || !warm) RF_HIP(rf::fill(n, 0.0, s->x, s->stream));
-  if (bnorm == 0.0) {
+  if (!warm) RF_HIP(rf::fill(n, 0.0, s->x, s->stream));
+  const double* first = s->b;
+  if (warm) {
+    first = r0x;
+    if (!first) {
+      RF_HIP(sim_gemv(s, s->x, s->gpart, r, s->b, 1));
+      first = r;
+    }
+  }
+  // The scalars live on the device, the start's included; the host stays one
+  // iteration ahead (it enqueues iteration k + 1, then waits for the control of
+  // iteration k, which it sees in pinned memory), and the kernels of an
+  // iteration enqueued after the end return at once.
+  const rf::BicgVecs w{s->x, r, p, v, sv};
+  const int launched0 = s->ngemv;
+  const volatile rf::SolveMirror* mir = s->mirror;
+  reset_mirror(s);
+  RF_HIP(rf::bicg_start(n, w, s->b, first, s->dpart, tol, s->bicg, s->stream));
+  for (int k = 0; k < maxit; ++k) {
+    if (k > 0) {  // a pending restart: r = b - A x (untimed), r0 = p = r, rho = ||r||^2
+      if (s->oper)
+        RF_HIP(rf::op_product(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->x, r,
+                              s->b, 1, s->pc, s->stream, nullptr, nullptr, &s->bicg.head->no_restart));
+      else if (s->theta)
+        RF_HIP(rf::gemv_theta(s->N, s->M, s->Lp, s->T, s->ori[s->cur], s->x, r, s->b, 1, s->pc, s->stream,
+                              nullptr, nullptr, &s->bicg.head->no_restart));
+      else
+        RF_HIP(rf::gemv(s->plan, s->A, s->x, s->gpart, r, s->b, 1, s->stream, nullptr, nullptr,
+                        &s->bicg.head->no_restart));
+      RF_HIP(rf::bicg_restart(n, w, s->dpart, s->bicg, s->stream));
+    }
+    RF_HIP(sim_gemv(s, p, s->gpart, v, nullptr, 0, false, &s->bicg.head->done));
+    RF_HIP(rf::bicg_after_v(n, k + 1, w, s->dpart, tol, s->bicg, s->stream));
+    RF_HIP(sim_gemv(s, sv, s->gpart, t, nullptr, 0, false, &s->bicg.head->done));
+    RF_HIP(rf::bicg_after_t(n, w, s->dpart, tol, s->bicg, s->stream));
+    if (k > 0) {
+      RF_TRY(wait_progress(s, k));
+      if (mir->done) break;
+    }
+  }
+  RF_TRY(wait_progress(s, maxit));
+  rf::BicgHead hd{};
+  if (!mir->done) {  // out of iterations
+    RF_HIP(hipMemcpyAsync(&hd, s->bicg.head, sizeof(hd), hipMemcpyDeviceToHost, s->stream));
+    RF_HIP(hipStreamSynchronize(s->stream));
+  }
+  if (mir->done) {  // by the iteration after whose progress the host looked, too
+    hd.its = mir->used;
+    hd.prods = mir->prods;
+    hd.restarts = mir->restarts;
+    hd.nonfinite = mir->nonfinite;
+    hd.converged = mir->converged;
+    hd.res = mir->res;
+    hd.bnorm = mir->bnorm;
+  }
+  s->ngemv = std::min(s->ngemv, launched0 + hd.prods);  // products that returned at once are not counted
+  s->bicg_restarts = hd.restarts;
+  if (hd.nonfinite == 2) return fail(RF_ERR_NONFINITE, "non-finite right-hand side");
+  if (hd.nonfinite) return fail(RF_ERR_NONFINITE, "non-finite residual in BiCGStab");
+  if (hd.bnorm == 0.0) {
+    RF_HIP(rf::fill(n, 0.0, s->x, s->stream));
     s->stats.converged = 1;
     return RF_OK;
   }
-  double rho, res;
-  if (warm) {
-    if (r0x)
-      RF_HIP(rf::axpby(n, 1.0, r0x, 0.0, r, s->stream));
-    else
-      RF_HIP(sim_gemv(s, s->x, s->gpart, r, s->b, 1));
-    RF_TRY(device_norm(s, r, &res));
-    rho = res * res;
-  } else {
-    RF_HIP(rf::axpby(n, 1.0, s->b, 0.0, r, s->stream));
-    rho = bnorm * bnorm;
-    res = bnorm;
-  }
-  RF_HIP(rf::axpby(n, 1.0, r, 0.0, r0, s->stream));
-  RF_HIP(rf::axpby(n, 1.0, r, 0.0, p, s->stream));
-  int it = 0;
-  bool converged = res / bnorm <= tol;
-  if (!converged && maxit > 0) {
-    // The scalars live on the device; the host stays one iteration ahead (it
-    // enqueues iteration k + 1, then waits for the end of iteration k and reads
-    // the done flag mirrored into host memory), and the kernels of an
-    // iteration enqueued after the end return at once.
-    const rf::BicgVecs w{s->x, r, p, v, sv};
-    const int launched0 = s->ngemv;
-    RF_HIP(rf::bicg_start(s->bicg, rho, res, s->stream));
-    for (int k = 0; k < maxit; ++k) {
-      if (k > 0) {  // a pending restart: r = b - A x (untimed), r0 = p = r, rho = ||r||^2
-        if (s->oper)
-          RF_HIP(rf::op_product(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->x, r,
-                                s->b, 1, s->pc, s->stream, nullptr, nullptr, &s->bicg.head->no_restart));
-        else if (s->theta)
-          RF_HIP(rf::gemv_theta(s->N, s->M, s->Lp, s->T, s->ori[s->cur], s->x, r, s->b, 1, s->pc, s->stream,
-                                nullptr, nullptr, &s->bicg.head->no_restart));
-        else
-          RF_HIP(rf::gemv(s->plan, s->A, s->x, s->gpart, r, s->b, 1, s->stream, nullptr, nullptr,
-                          &s->bicg.head->no_restart));
-        RF_HIP(rf::bicg_restart(n, w, s->dpart, s->bicg, s->stream));
-      }
-      RF_HIP(sim_gemv(s, p, s->gpart, v, nullptr, 0, false, &s->bicg.head->done));
-      RF_HIP(rf::bicg_after_v(n, k + 1, w, s->dpart, tol, bnorm, s->bicg, s->stream));
-      RF_HIP(sim_gemv(s, sv, s->gpart, t, nullptr, 0, false, &s->bicg.head->done));
-      RF_HIP(rf::bicg_after_t(n, w, s->dpart, tol, bnorm, s->bicg, s->stream));
-      RF_HIP(hipEventRecord(s->cev[k & 1], s->stream));
-      if (k > 0) {
-        RF_HIP(hipEventSynchronize(s->cev[(k - 1) & 1]));
-        if (*static_cast<volatile int*>(s->hdone)) break;
-      }
-    }
-    rf::BicgHead hd{};
-    RF_HIP(hipMemcpyAsync(&hd, s->bicg.head, sizeof(hd), hipMemcpyDeviceToHost, s->stream));
-    RF_HIP(hipStreamSynchronize(s->stream));
-    s->ngemv = std::min(s->ngemv, launched0 + hd.prods);  // products that returned at once are not counted
-    s->bicg_restarts = hd.restarts;
-    if (hd.nonfinite) return fail(RF_ERR_NONFINITE, "non-finite residual in BiCGStab");
-    it = hd.its;
-    converged = hd.converged != 0;
-    res = hd.res;
-  }
+  const int it = hd.its;
+  bool converged = hd.converged != 0;
+  double res = hd.res;
+  const double bnorm = hd.bnorm;
   // A converged solve reports its recurrence residual, as the reference's
   // solver does (lib/viennacl/linalg/bicgstab.hpp:146-148,160); the true
   // residual of the returned x when it did not converge, or on request.
@@ -788,15 +803,17 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
   if (hipGetDevice(&s->device) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "no HIP device"));
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
     return cleanup(fail(RF_ERR_DEVICE, "hipStreamCreate failed"));
+  // Timing events: no system-scope fence, which halves what a recorded event
+  // costs a chain of small kernels (a step at M = 100: 0.387 with, 0.359 without,
+  // 0.339 ms with no event at all); what the host reads without a copy, the
+  // kernels fence themselves.  ev[4] ends the step and keeps the fence.
   for (auto& e : s->ev)
-    if (hipEventCreate(&e) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
+    if ((&e == &s->ev[4] ? hipEventCreate(&e) : hipEventCreateWithFlags(&e, hipEventDisableSystemFence)) !=
+        hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
   for (auto& e : s->gev)
-    if (hipEventCreate(&e) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
+    if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
   for (auto& e : s->hev)
-    if (hipEventCreate(&e) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
-  for (auto& e : s->cev)
-    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
-      return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
+    if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "hipEventCreate failed"));
 
   const int64_t n = s->n;
   const size_t fiber3 = 3 * static_cast<size_t>(M);
@@ -889,22 +906,24 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
     }
     void* hp = nullptr;
     void* dp = nullptr;
-    if (st == RF_OK && (hipHostMalloc(&hp, 64, hipHostMallocMapped) != hipSuccess ||
+    static_assert(sizeof(rf::SolveMirror) <= 128, "the pinned block's layout");
+    if (st == RF_OK && (hipHostMalloc(&hp, 256, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
                         hipHostGetDevicePointer(&dp, hp, 0) != hipSuccess)) {
       if (hp) (void)hipHostFree(hp);
       (void)hipGetLastError();
-      st = fail(RF_ERR_OUT_OF_MEMORY, "hipHostMalloc of the solver's done flag failed");
+      st = fail(RF_ERR_OUT_OF_MEMORY, "hipHostMalloc of the solver's mirror failed");
     } else if (st == RF_OK) {
-      s->hdone = static_cast<int*>(hp);
-      s->near_used = static_cast<unsigned long long*>(hp) + 2;
-      *s->hdone = 0;
-      s->cyc.hdone = static_cast<int*>(dp);
-      s->bicg.hdone = static_cast<int*>(dp);
+      std::memset(hp, 0, 256);
+      s->mirror = static_cast<rf::SolveMirror*>(hp);
+      s->near_used = reinterpret_cast<unsigned long long*>(static_cast<char*>(hp) + 128);
+      s->nonfinite = reinterpret_cast<int*>(static_cast<char*>(hp) + 192);
+      s->nonfinite_dev = reinterpret_cast<int*>(static_cast<char*>(dp) + 192);
+      s->cyc.mirror = static_cast<rf::SolveMirror*>(dp);
+      s->bicg.mirror = static_cast<rf::SolveMirror*>(dp);
     }
   }
   if (st == RF_OK) st = s->alloc(&s->dpart, dpart_len);
   if (st == RF_OK) st = s->alloc(&s->hdev, static_cast<size_t>(2 * kmax + 4));
-  if (st == RF_OK) st = s->alloc(&s->flag, 1);
   if (st != RF_OK) return cleanup(st);
   if (cfg->solver == RF_SOLVER_DIRECT || cfg->solver == RF_SOLVER_DIRECT_MIXED_BF16 ||
       cfg->solver == RF_SOLVER_DIRECT_MIXED_FP16) {
@@ -942,9 +961,7 @@ void rf_destroy(rf_simulation* s) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : s->hev)
     if (e) (void)hipEventDestroy(e);
-  for (auto& e : s->cev)
-    if (e) (void)hipEventDestroy(e);
-  if (s->hdone) (void)hipHostFree(s->hdone);
+  if (s->mirror) (void)hipHostFree(s->mirror);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   delete s;
 }
@@ -1062,10 +1079,20 @@ rf_status rf_step(rf_simulation* s, int64_t current_timestep) {
   RF_HIP(hipEventRecord(s->ev[2], s->stream));
   RF_TRY(rf_update_velocities(s));
   RF_HIP(hipEventRecord(s->ev[3], s->stream));
-  RF_TRY(check_nonfinite(s, s->tv[s->vcur], 3LL * s->M, "translational velocities"));
+  // The update is enqueued before the check of the velocities it takes is read:
+  // non-finite ones make the next state's buffers worthless, which are then
+  // not advanced to.
+  const int old_plast = s->plast;
+  *s->nonfinite = 0;
+  RF_HIP(rf::nonfinite_count(3LL * s->M, s->tv[s->vcur], s->nonfinite_dev, s->stream));
   RF_TRY(rf_update_fibers(s, current_timestep == 0 ? 1 : 0));
   RF_HIP(hipEventRecord(s->ev[4], s->stream));
   RF_HIP(hipEventSynchronize(s->ev[4]));
+  if (*static_cast<volatile int*>(s->nonfinite)) {
+    s->have_next = false;
+    s->plast = old_plast;
+    return fail(RF_ERR_NONFINITE, "non-finite values in translational velocities");
+  }
   s->timings.assemble_system = elapsed(s->ev[0], s->ev[1]);
   s->timings.solve_system = elapsed(s->ev[1], s->ev[2]);
   s->timings.update_velocities = elapsed(s->ev[2], s->ev[3]);

@@ -259,18 +259,35 @@ hipError_t mdot(int64_t n, int K, const double* V, int64_t ldv, const double* w,
 // y = alpha * x + beta * y
 hipError_t axpby(int64_t n, double alpha, const double* x, double beta, double* y, hipStream_t s);
 hipError_t fill(int64_t n, double value, double* y, hipStream_t s);
-hipError_t nonfinite_count(int64_t n, const double* x, int* flag_dev, hipStream_t s);
+// *flag (device address of host or device memory) = 1 if x has a non-finite value.
+hipError_t nonfinite_count(int64_t n, const double* x, int* flag, hipStream_t s);
+
+// What the host sees of a solve while it runs: pinned host memory that the
+// device control writes.  done is written last; progress counts the steps (or
+// iterations) whose control has run.
+struct SolveMirror {
+  int done;
+  int progress;
+  int used;       // GMRES: Arnoldi steps of the cycle; BiCGStab: iterations
+  int nonfinite;  // 1: a vector of the iteration, 2: the right-hand side, 3: the first residual
+  int start;      // how the solve's (or cycle's) start ended it: 1 zero right-hand side, 2 tolerance met
+  int converged;  // BiCGStab
+  int prods;      // BiCGStab: products that ran
+  int restarts;   // BiCGStab
+  double res, bnorm;
+};
 
 // One restart cycle of single-simulation GMRES(m) with its control on the
-// device (rf_linalg.hip): the step that ends the cycle sets head.done (and
-// *hdone in host memory), and the products and vector kernels of steps
-// enqueued later return at once.
+// device (rf_linalg.hip): the start or the step that ends the cycle sets
+// head.done, and the products and vector kernels of steps enqueued later
+// return at once.
 struct CycleHead {
   int done;       // the cycle has ended
   int k_used;     // its Arnoldi steps
-  int nonfinite;  // a non-finite ||w|| ended it
-  int pad;
+  int nonfinite;  // as SolveMirror
+  int start;      // as SolveMirror
   double res;     // |g_k|, the cycle's residual estimate
+  double bnorm;   // ||b||
 };
 struct CycleCtl {
   CycleHead* head;
@@ -279,21 +296,24 @@ struct CycleCtl {
   double* sn;
   double* g;  // m + 1
   double* y;  // m
-  int* hdone;  // pinned host memory (device address): head.done mirrored
+  SolveMirror* mirror;  // device address
 };
 // Device doubles of a cycle's control (head included), and its layout in them.
 size_t cycle_ctl_doubles(int m);
 CycleCtl cycle_ctl(double* mem, int m);
 // Dot partials of the steps.
 size_t cycle_part_doubles(int64_t n, int m);
-// g = (beta, 0, ..., 0), head cleared.
-hipError_t cycle_start(const CycleCtl& c, int m, double beta, hipStream_t s);
+// Start of a cycle from the residual r: ||b||, beta = ||r||, V_0 = r / beta (V_0
+// may be r), g = (beta, 0, ..., 0), head cleared.  A non-finite norm, b = 0 or
+// beta <= tol ||b|| ends the cycle there.
+hipError_t cycle_start(int64_t n, const CycleCtl& c, int m, const double* b, const double* r, double* V0, double* part,
+                       double tol, hipStream_t s);
 // Step k on w = A V_k (= V_{k+1}, V column stride n): Gram-Schmidt twice
 // against V_0..V_k, the Hessenberg column and its Givens rotation, and the
 // end test ||r|| <= tol ||b||, a breakdown ||w|| = 0 or k = klast, where
 // y = H^-1 g is formed; else w /= ||w||.
 hipError_t arnoldi_step(int64_t n, int k, int klast, int m, const double* V, double* w, double* part, double tol,
-                        double bnorm, const CycleCtl& c, hipStream_t s);
+                        const CycleCtl& c, hipStream_t s);
 // x += sum_{k < k_used} V_k y_k
 hipError_t cycle_update(int64_t n, const double* V, const CycleCtl& c, double* x, hipStream_t s);
 
@@ -312,11 +332,11 @@ struct BicgHead {
   int no_restart; // 1 unless a restart is pending and the solve goes on (the skip flag of the restart's kernels)
   int last_restart;  // iteration of the last restart (the start counts as one)
   int restarts;      // restarts so far
-  double rho, alpha, omega, beta, res;
+  double rho, alpha, omega, beta, res, bnorm;
 };
 struct BicgCtl {
   BicgHead* head;
-  int* hdone;  // pinned host memory (device address): head.done mirrored
+  SolveMirror* mirror;  // device address
 };
 struct BicgVecs {
   double* x;
@@ -326,17 +346,19 @@ struct BicgVecs {
   double* s;   // t follows s at stride n
 };
 size_t bicg_part_doubles(int64_t n);
-hipError_t bicg_start(const BicgCtl& c, double rho, double res, hipStream_t s);
+// Start from the residual r0 (copied to w.r and its followers r0 and p): ||b||,
+// rho = ||r||^2; a non-finite norm, b = 0 or ||r|| <= tol ||b|| ends it there.
+hipError_t bicg_start(int64_t n, const BicgVecs& w, const double* b, const double* r0, double* part, double tol,
+                      const BicgCtl& c, hipStream_t s);
 // A pending restart (lib/viennacl/linalg/bicgstab.hpp:119-131): after the
 // caller's r = b - A x (a product skipped unless head.no_restart is 0),
 // r0 = p = r and rho = ||r||^2; nothing when no restart is pending.
 hipError_t bicg_restart(int64_t n, const BicgVecs& w, double* part, const BicgCtl& c, hipStream_t s);
 // After v = A p of iteration it (1-based): alpha, s = r - alpha v, ||s||
 // and the early end with x += alpha p.
-hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, double tol, double bnorm,
-                        const BicgCtl& c, hipStream_t s);
-// After t = A s: omega, x and r, ||r|| and <r0, r>, the end test, p.
-hipError_t bicg_after_t(int64_t n, const BicgVecs& w, double* part, double tol, double bnorm, const BicgCtl& c,
+hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, double tol, const BicgCtl& c,
                         hipStream_t s);
+// After t = A s: omega, x and r, ||r|| and <r0, r>, the end test, p.
+hipError_t bicg_after_t(int64_t n, const BicgVecs& w, double* part, double tol, const BicgCtl& c, hipStream_t s);
 
 }  // namespace rf

@@ -354,12 +354,14 @@ hipError_t fill(int64_t n, double value, double* y, hipStream_t s) {
 
 __global__ void nonfinite_kernel(int64_t n, const double* __restrict__ x, int* __restrict__ flag) {
   const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (r < n && !isfinite(x[r])) flag[0] = 1;  // benign race: any writer stores 1
+  if (r < n && !isfinite(x[r])) {
+    *const_cast<volatile int*>(flag) = 1;  // benign race: any writer stores 1
+    __threadfence_system();
+  }
 }
 
-hipError_t nonfinite_count(int64_t n, const double* x, int* flag_dev, hipStream_t s) {
-  hipLaunchKernelGGL(nonfinite_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, n, x,
-                     flag_dev);
+hipError_t nonfinite_count(int64_t n, const double* x, int* flag, hipStream_t s) {
+  hipLaunchKernelGGL(nonfinite_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, n, x, flag);
   return hipGetLastError();
 }
 
@@ -842,7 +844,7 @@ CycleCtl cycle_ctl(double* mem, int m) {
   c.sn = c.cs + m;
   c.g = c.sn + m;
   c.y = c.g + m + 1;
-  c.hdone = nullptr;
+  c.mirror = nullptr;
   return c;
 }
 
@@ -857,16 +859,32 @@ static int pass_blocks(int64_t n) { return static_cast<int>((n + pass_rows(n) - 
 
 size_t cycle_part_doubles(int64_t n, int m) { return 3 * static_cast<size_t>(m + 1) * pass_blocks(n); }
 
-__global__ void cycle_start_kernel(CycleCtl c, int m, double beta) {
-  for (int i = threadIdx.x; i <= m; i += blockDim.x) c.g[i] = (i == 0) ? beta : 0.0;
-  if (threadIdx.x == 0) {
-    c.head->done = 0;
-    c.head->k_used = 0;
-    c.head->nonfinite = 0;
-    c.head->pad = 0;
-    c.head->res = beta;
-    if (c.hdone) *c.hdone = 0;
-  }
+// The head to the host, done last.
+__device__ __forceinline__ void cycle_publish(const CycleCtl& c) {
+  const CycleHead& h = *c.head;
+  SolveMirror* m = c.mirror;
+  m->used = h.k_used;
+  m->nonfinite = h.nonfinite;
+  m->start = h.start;
+  m->res = h.res;
+  m->bnorm = h.bnorm;
+  __threadfence_system();
+  *const_cast<volatile int*>(&m->done) = h.done;
+}
+
+// The control of a cycle's start, by one lane.
+__device__ __forceinline__ void cycle_start_control(double b2, double r2, int m, double tol, const CycleCtl& c) {
+  CycleHead& h = *c.head;
+  const double bnorm = sqrt(b2), beta = sqrt(r2);
+  for (int i = 1; i <= m; ++i) c.g[i] = 0.0;
+  c.g[0] = beta;
+  h.k_used = 0;
+  h.bnorm = bnorm;
+  h.res = beta;
+  h.nonfinite = !isfinite(bnorm) ? 2 : (bnorm != 0.0 && !isfinite(beta) ? 3 : 0);
+  h.start = h.nonfinite ? 0 : (bnorm == 0.0 ? 1 : (beta / bnorm <= tol ? 2 : 0));
+  h.done = h.nonfinite != 0 || h.start != 0;
+  cycle_publish(c);
 }
 
 // Sum of one reduction's block partials by the lanes of a wavefront (every lane
@@ -947,7 +965,7 @@ __global__ __launch_bounds__(256) void arnoldi_pass_kernel(int64_t n, int64_t ro
 // The control of step k, by one lane: H(:, k) = h0 + h1 and ||w||, the earlier
 // rotations and a new one, g and the estimate |g_{k+1}|; at the cycle's end
 // y = H^-1 g.  hs: h0[K], h1[K], ||w||^2.
-__device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const double* hs, double tol, double bnorm,
+__device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const double* hs, double tol,
                                                 const CycleCtl& c) {
   CycleHead& hd = *c.head;
   const int K = k + 1;
@@ -956,7 +974,7 @@ __device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const d
     hd.nonfinite = 1;
     hd.k_used = k;
     hd.done = 1;
-    if (c.hdone) *c.hdone = 1;
+    cycle_publish(c);
     return;
   }
   double* Hk = c.H + static_cast<int64_t>(k) * (m + 1);
@@ -977,7 +995,7 @@ __device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const d
   c.g[k] = c.cs[k] * c.g[k];
   const double res = fabs(c.g[k + 1]);
   hd.res = res;
-  if (res / bnorm <= tol || hn == 0.0 || k == klast) {
+  if (res / hd.bnorm <= tol || hn == 0.0 || k == klast) {
     for (int i = k; i >= 0; --i) {
       double acc = c.g[i];
       for (int j = i + 1; j <= k; ++j) acc -= c.H[i + static_cast<int64_t>(j) * (m + 1)] * c.y[j];
@@ -985,7 +1003,9 @@ __device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const d
     }
     hd.k_used = K;
     hd.done = 1;
-    if (c.hdone) *c.hdone = 1;
+    cycle_publish(c);
+  } else {
+    *const_cast<volatile int*>(&c.mirror->progress) = K;  // never after done: the host may have begun the next cycle
   }
 }
 
@@ -993,8 +1013,7 @@ __device__ __forceinline__ void arnoldi_control(int k, int klast, int m, const d
 // starts after it ended the cycle returns: the vector is not read any more).
 __global__ __launch_bounds__(256) void arnoldi_finish_kernel(int64_t n, int nb, int k, int klast, int m,
                                                              int64_t region, const double* __restrict__ part,
-                                                             double* __restrict__ w, double tol, double bnorm,
-                                                             CycleCtl c) {
+                                                             double* __restrict__ w, double tol, CycleCtl c) {
   extern __shared__ double hs[];  // first workgroup: h0[K], h1[K], ||w||^2
   if (c.head->done) return;
   const int K = k + 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1009,7 +1028,7 @@ __global__ __launch_bounds__(256) void arnoldi_finish_kernel(int64_t n, int nb, 
     if (lane == 0) hs[t] = v;
   }
   __syncthreads();
-  if (threadIdx.x == 0) arnoldi_control(k, klast, m, hs, tol, bnorm, c);
+  if (threadIdx.x == 0) arnoldi_control(k, klast, m, hs, tol, c);
 }
 
 // The whole step in one workgroup: w in registers, each Gram-Schmidt pass's
@@ -1019,7 +1038,7 @@ constexpr int kOneGroupRows = 8192;   // 8 per lane
 constexpr int kOneGroupWork = 65536;  // n K: beyond it one CU's loads of V take longer than the launches
 __global__ __launch_bounds__(kOneGroup) void arnoldi_one_kernel(int n, int k, int klast, int m,
                                                                 const double* __restrict__ V, double* __restrict__ w,
-                                                                double tol, double bnorm, CycleCtl c) {
+                                                                double tol, CycleCtl c) {
   constexpr int R = kOneGroupRows / kOneGroup, W = kOneGroup / 64;
   extern __shared__ double hs[];  // h0[K], h1[K], ||w||^2
   __shared__ double red[W][kPassChunk];
@@ -1093,12 +1112,12 @@ __global__ __launch_bounds__(kOneGroup) void arnoldi_one_kernel(int n, int k, in
     const int r = static_cast<int>(threadIdx.x) + e * kOneGroup;
     if (r < n) w[r] = scale * wr[e];
   }
-  if (threadIdx.x == 0) arnoldi_control(k, klast, m, hs, tol, bnorm, c);
+  if (threadIdx.x == 0) arnoldi_control(k, klast, m, hs, tol, c);
 }
 
 __global__ void cycle_update_kernel(int64_t n, const double* __restrict__ V, CycleCtl c, double* __restrict__ x) {
   const int K = c.head->k_used;
-  if (c.head->nonfinite) return;
+  if (c.head->nonfinite || K == 0) return;
   const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (r >= n) return;
   double s = 0.0;
@@ -1106,19 +1125,102 @@ __global__ void cycle_update_kernel(int64_t n, const double* __restrict__ V, Cyc
   x[r] = fma(1.0, s, x[r]);
 }
 
-hipError_t cycle_start(const CycleCtl& c, int m, double beta, hipStream_t s) {
-  hipLaunchKernelGGL(cycle_start_kernel, dim3(1), dim3(64), 0, s, c, m, beta);
+// Sums over the workgroup of kOneGroup lanes, every lane returning them.
+template <int S>
+__device__ __forceinline__ void one_group_sums(double (&d)[S], double (*red)[2]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) d[q] += __shfl_xor(d[q], off, 64);
+    if (lane == 0) red[wave][q] = d[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < S; ++q) {
+    d[q] = 0.0;
+#pragma unroll
+    for (int v = 0; v < kOneGroup / 64; ++v) d[q] += red[v][q];
+  }
+  __syncthreads();
+}
+
+// A cycle's start in one workgroup (n <= kOneGroupRows).
+__global__ __launch_bounds__(kOneGroup) void cycle_start_one_kernel(int n, int m, const double* __restrict__ b,
+                                                                    const double* r, double* V0, double tol,
+                                                                    CycleCtl c) {
+  constexpr int R = kOneGroupRows / kOneGroup;
+  __shared__ double red[kOneGroup / 64][2];
+  double v[R], d[2] = {0.0, 0.0};
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    v[e] = i < n ? r[i] : 0.0;
+    const double bi = i < n ? b[i] : 0.0;
+    d[0] = fma(bi, bi, d[0]);
+    d[1] = fma(v[e], v[e], d[1]);
+  }
+  one_group_sums<2>(d, red);
+  const double scale = 1.0 / sqrt(d[1]);
+#pragma unroll
+  for (int e = 0; e < R; ++e) {
+    const int i = static_cast<int>(threadIdx.x) + e * kOneGroup;
+    if (i < n) V0[i] = scale * v[e];
+  }
+  if (threadIdx.x == 0) cycle_start_control(d[0], d[1], m, tol, c);
+}
+
+// Partials of ||b||^2 (part[block]) and ||r||^2 (part[nb + block]).
+__global__ __launch_bounds__(256) void norms_kernel(int64_t n, int64_t rows, const double* __restrict__ b,
+                                                    const double* __restrict__ r, double* __restrict__ part) {
+  __shared__ double sh[4];
+  const int64_t lo = static_cast<int64_t>(blockIdx.x) * rows, hi = min(n, lo + rows);
+  double b2 = 0.0, r2 = 0.0;
+  for (int64_t i = lo + threadIdx.x; i < hi; i += 256) {
+    b2 = fma(b[i], b[i], b2);
+    r2 = fma(r[i], r[i], r2);
+  }
+  const double sb = block_sum(b2, sh);
+  __syncthreads();
+  const double sr = block_sum(r2, sh);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = sb;
+    part[gridDim.x + blockIdx.x] = sr;
+  }
+}
+
+__global__ __launch_bounds__(256) void cycle_start_kernel(int64_t n, int nb, int m, const double* __restrict__ part,
+                                                          const double* r, double* V0, double tol, CycleCtl c) {
+  const double r2 = wave_sum(part + nb, nb);
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) V0[i] = (1.0 / sqrt(r2)) * r[i];
+  if (blockIdx.x != 0 || threadIdx.x >= 64) return;
+  const double b2 = wave_sum(part, nb);
+  if (threadIdx.x == 0) cycle_start_control(b2, r2, m, tol, c);
+}
+
+hipError_t cycle_start(int64_t n, const CycleCtl& c, int m, const double* b, const double* r, double* V0, double* part,
+                       double tol, hipStream_t s) {
+  if (n <= kOneGroupRows) {
+    hipLaunchKernelGGL(cycle_start_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), m, b, r, V0, tol,
+                       c);
+    return hipGetLastError();
+  }
+  const int nb = pass_blocks(n);
+  hipLaunchKernelGGL(norms_kernel, dim3(nb), dim3(256), 0, s, n, pass_rows(n), b, r, part);
+  hipLaunchKernelGGL(cycle_start_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, n, nb, m,
+                     static_cast<const double*>(part), r, V0, tol, c);
   return hipGetLastError();
 }
 
 hipError_t arnoldi_step(int64_t n, int k, int klast, int m, const double* V, double* w, double* part, double tol,
-                        double bnorm, const CycleCtl& c, hipStream_t s) {
+                        const CycleCtl& c, hipStream_t s) {
   if (k < 0 || k > klast || klast >= m) return hipErrorInvalidValue;
   const int K = k + 1;
   const size_t hbytes = (2 * static_cast<size_t>(K) + 1) * sizeof(double);
   if (n <= kOneGroupRows && n * K <= kOneGroupWork) {
     hipLaunchKernelGGL(arnoldi_one_kernel, dim3(1), dim3(kOneGroup), hbytes, s, static_cast<int>(n), k, klast, m, V, w,
-                       tol, bnorm, c);
+                       tol, c);
     return hipGetLastError();
   }
   const int64_t rows = pass_rows(n);
@@ -1130,7 +1232,7 @@ hipError_t arnoldi_step(int64_t n, int k, int klast, int m, const double* V, dou
     hipLaunchKernelGGL(arnoldi_pass_kernel, dim3(nb), dim3(256), pbytes, s, n, rows, phase, K, region, V, w, part,
                        skip);
   hipLaunchKernelGGL(arnoldi_finish_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), hbytes, s, n, nb,
-                     k, klast, m, region, static_cast<const double*>(part), w, tol, bnorm, c);
+                     k, klast, m, region, static_cast<const double*>(part), w, tol, c);
   return hipGetLastError();
 }
 
@@ -1147,7 +1249,10 @@ hipError_t cycle_update(int64_t n, const double* V, const CycleCtl& c, double* x
 // kOneGroupRows: one workgroup does what follows each product, in one launch
 // instead of six.
 
-size_t bicg_part_doubles(int64_t n) { return 6 * static_cast<size_t>(mdot_blocks(n)); }
+size_t bicg_part_doubles(int64_t n) {
+  const size_t iteration = 6 * static_cast<size_t>(mdot_blocks(n)), start = 2 * static_cast<size_t>(pass_blocks(n));
+  return iteration > start ? iteration : start;
+}
 
 __device__ __forceinline__ double wave_sum_parts(const double* __restrict__ part, int nb) {
   double s = 0.0;
@@ -1157,18 +1262,29 @@ __device__ __forceinline__ double wave_sum_parts(const double* __restrict__ part
   return s;
 }
 
+// The solve's end: the head to the host, done last.
 __device__ __forceinline__ void bicg_end(const BicgCtl& c) {
-  c.head->done = 1;
-  c.head->no_restart = 1;
-  if (c.hdone) *c.hdone = 1;
+  BicgHead& h = *c.head;
+  h.done = 1;
+  h.no_restart = 1;
+  SolveMirror* m = c.mirror;
+  m->used = h.its;
+  m->nonfinite = h.nonfinite;
+  m->converged = h.converged;
+  m->prods = h.prods;
+  m->restarts = h.restarts;
+  m->res = h.res;
+  m->bnorm = h.bnorm;
+  __threadfence_system();
+  *const_cast<volatile int*>(&m->done) = 1;
 }
 
 // Iterations after which BiCGStab restarts from the true residual
 // (max_iterations_before_restart, lib/viennacl/linalg/bicgstab.hpp:52).
 constexpr int kBicgRestartEvery = 200;
 
-__global__ void bicg_start_kernel(BicgCtl c, double rho, double res) {
-  if (threadIdx.x != 0) return;
+// The control of a solve's start, by one lane.
+__device__ __forceinline__ void bicg_start_control(double b2, double r2, double tol, const BicgCtl& c) {
   BicgHead& h = *c.head;
   h.done = 0;
   h.converged = 0;
@@ -1180,10 +1296,56 @@ __global__ void bicg_start_kernel(BicgCtl c, double rho, double res) {
   h.no_restart = 1;
   h.last_restart = 0;
   h.restarts = 0;
-  h.rho = rho;
+  h.bnorm = sqrt(b2);
+  h.res = sqrt(r2);
+  h.rho = h.res * h.res;
   h.alpha = h.omega = h.beta = 0.0;
-  h.res = res;
-  if (c.hdone) *c.hdone = 0;
+  c.mirror->start = 0;
+  if (!isfinite(h.bnorm)) {
+    h.nonfinite = 2;
+    bicg_end(c);
+  } else if (h.bnorm == 0.0) {
+    c.mirror->start = 1;
+    h.converged = 1;
+    bicg_end(c);
+  } else if (!isfinite(h.res)) {
+    h.nonfinite = 3;
+    bicg_end(c);
+  } else if (h.res / h.bnorm <= tol) {
+    c.mirror->start = 2;
+    h.converged = 1;
+    bicg_end(c);
+  }
+}
+
+__global__ __launch_bounds__(kOneGroup) void bicg_start_one_kernel(int n, BicgVecs w, const double* __restrict__ b,
+                                                                   const double* r0, double tol, BicgCtl c) {
+  __shared__ double red[kOneGroup / 64][2];
+  double d[2] = {0.0, 0.0};
+  for (int i = threadIdx.x; i < n; i += kOneGroup) {
+    const double ri = r0[i], bi = b[i];
+    w.r[i] = ri;
+    w.r[n + i] = ri;
+    w.p[i] = ri;
+    d[0] = fma(bi, bi, d[0]);
+    d[1] = fma(ri, ri, d[1]);
+  }
+  one_group_sums<2>(d, red);
+  if (threadIdx.x == 0) bicg_start_control(d[0], d[1], tol, c);
+}
+
+__global__ __launch_bounds__(256) void bicg_start_kernel(int64_t n, int nb, const double* __restrict__ part, BicgVecs w,
+                                                         const double* r0, double tol, BicgCtl c) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i < n) {
+    const double ri = r0[i];
+    w.r[i] = ri;
+    w.r[n + i] = ri;
+    w.p[i] = ri;
+  }
+  if (blockIdx.x != 0 || threadIdx.x >= 64) return;
+  const double b2 = wave_sum(part, nb), r2 = wave_sum(part + nb, nb);
+  if (threadIdx.x == 0) bicg_start_control(b2, r2, tol, c);
 }
 
 // alpha = rho / <r0, v>; a zero or non-finite <r0, v> ends the solve
@@ -1210,7 +1372,7 @@ __global__ void bicg_s_kernel(int64_t n, const double* __restrict__ r, const dou
 }
 
 __global__ __launch_bounds__(64) void bicg_snorm_kernel(int it, int nb, const double* __restrict__ part, double tol,
-                                                        double bnorm, BicgCtl c) {
+                                                        BicgCtl c) {
   BicgHead& h = *c.head;
   if (h.done) return;
   const double snorm = sqrt(wave_sum_parts(part, nb));
@@ -1218,7 +1380,7 @@ __global__ __launch_bounds__(64) void bicg_snorm_kernel(int it, int nb, const do
   if (!isfinite(snorm)) {
     h.nonfinite = 1;
     bicg_end(c);
-  } else if (snorm / bnorm <= tol) {
+  } else if (snorm / h.bnorm <= tol) {
     h.res = snorm;
     h.converged = 1;
     h.early_it = it;
@@ -1261,19 +1423,21 @@ __global__ void bicg_xr_kernel(int64_t n, const double* __restrict__ p, const do
 // iterations since the last restart sets up a restart from the true residual
 // at the next iteration (lib/viennacl/linalg/bicgstab.hpp:150-152).
 __global__ __launch_bounds__(64) void bicg_end_kernel(int nb, const double* __restrict__ part, double tol,
-                                                      double bnorm, BicgCtl c) {
+                                                      BicgCtl c) {
   BicgHead& h = *c.head;
   if (h.done) return;
   const double rr = wave_sum_parts(part, nb), rho_new = wave_sum_parts(part + nb, nb);
   if (threadIdx.x != 0) return;
   const double res = sqrt(rr);
   h.res = res;
+  // its end, if this is one, is fenced after it
+  *const_cast<volatile int*>(&c.mirror->progress) = h.its;
   if (!isfinite(res)) {
     h.nonfinite = 1;
     bicg_end(c);
     return;
   }
-  if (res / bnorm <= tol) {
+  if (res / h.bnorm <= tol) {
     h.converged = 1;
     bicg_end(c);
     return;
@@ -1325,39 +1489,14 @@ __global__ __launch_bounds__(64) void bicg_restart_kernel(int nb, const double* 
   }
 }
 
-hipError_t bicg_start(const BicgCtl& c, double rho, double res, hipStream_t s) {
-  hipLaunchKernelGGL(bicg_start_kernel, dim3(1), dim3(64), 0, s, c, rho, res);
-  return hipGetLastError();
-}
-
-// Sums over the workgroup of kOneGroup lanes, every lane returning them.
-template <int S>
-__device__ __forceinline__ void one_group_sums(double (&d)[S], double (*red)[2]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int q = 0; q < S; ++q) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) d[q] += __shfl_xor(d[q], off, 64);
-    if (lane == 0) red[wave][q] = d[q];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < S; ++q) {
-    d[q] = 0.0;
-#pragma unroll
-    for (int v = 0; v < kOneGroup / 64; ++v) d[q] += red[v][q];
-  }
-  __syncthreads();
-}
 
 // What follows v = A p (bicg_alpha, _s, _snorm, _early) in one workgroup.
-__global__ __launch_bounds__(kOneGroup) void bicg_v_one_kernel(int n, int it, BicgVecs w, double tol, double bnorm,
-                                                               BicgCtl c) {
+__global__ __launch_bounds__(kOneGroup) void bicg_v_one_kernel(int n, int it, BicgVecs w, double tol, BicgCtl c) {
   constexpr int R = kOneGroupRows / kOneGroup;
   __shared__ double red[kOneGroup / 64][2];
   BicgHead& h = *c.head;
   if (h.done) return;
-  const double rho = h.rho;
+  const double rho = h.rho, bnorm = h.bnorm;
   const double* r0 = w.r + n;
   double v[R], r[R], d[1] = {0.0};
 #pragma unroll
@@ -1408,13 +1547,12 @@ __global__ __launch_bounds__(kOneGroup) void bicg_v_one_kernel(int n, int it, Bi
 }
 
 // What follows t = A s (bicg_omega, _xr, _end, _p) in one workgroup.
-__global__ __launch_bounds__(kOneGroup) void bicg_t_one_kernel(int n, BicgVecs w, double tol, double bnorm,
-                                                               BicgCtl c) {
+__global__ __launch_bounds__(kOneGroup) void bicg_t_one_kernel(int n, BicgVecs w, double tol, BicgCtl c) {
   constexpr int R = kOneGroupRows / kOneGroup;
   __shared__ double red[kOneGroup / 64][2];
   BicgHead& h = *c.head;
   if (h.done) return;
-  const double alpha = h.alpha, rho = h.rho;
+  const double alpha = h.alpha, rho = h.rho, bnorm = h.bnorm;
   const int since = h.its - 1 - h.last_restart;
   const double* r0 = w.r + n;
   const double* t = w.s + n;
@@ -1465,6 +1603,7 @@ __global__ __launch_bounds__(kOneGroup) void bicg_t_one_kernel(int n, BicgVecs w
       h.beta = beta;
       h.rho = rho_new;
     }
+    if (!bad && !met) *const_cast<volatile int*>(&c.mirror->progress) = h.its;
   }
   if (bad || met || restart) return;
 #pragma unroll
@@ -1503,6 +1642,19 @@ __global__ __launch_bounds__(kOneGroup) void bicg_restart_one_kernel(int n, Bicg
   }
 }
 
+hipError_t bicg_start(int64_t n, const BicgVecs& w, const double* b, const double* r0, double* part, double tol,
+                      const BicgCtl& c, hipStream_t s) {
+  if (n <= kOneGroupRows) {
+    hipLaunchKernelGGL(bicg_start_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), w, b, r0, tol, c);
+    return hipGetLastError();
+  }
+  const int nb = pass_blocks(n);
+  hipLaunchKernelGGL(norms_kernel, dim3(nb), dim3(256), 0, s, n, pass_rows(n), b, r0, part);
+  hipLaunchKernelGGL(bicg_start_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, n, nb,
+                     static_cast<const double*>(part), w, r0, tol, c);
+  return hipGetLastError();
+}
+
 hipError_t bicg_restart(int64_t n, const BicgVecs& w, double* part, const BicgCtl& c, hipStream_t s) {
   if (n <= kOneGroupRows) {
     hipLaunchKernelGGL(bicg_restart_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), w, c);
@@ -1518,10 +1670,10 @@ hipError_t bicg_restart(int64_t n, const BicgVecs& w, double* part, const BicgCt
   return hipGetLastError();
 }
 
-hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, double tol, double bnorm,
-                        const BicgCtl& c, hipStream_t s) {
+hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, double tol, const BicgCtl& c,
+                        hipStream_t s) {
   if (n <= kOneGroupRows) {
-    hipLaunchKernelGGL(bicg_v_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), it, w, tol, bnorm, c);
+    hipLaunchKernelGGL(bicg_v_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), it, w, tol, c);
     return hipGetLastError();
   }
   const int nb = mdot_blocks(n);
@@ -1535,15 +1687,14 @@ hipError_t bicg_after_v(int64_t n, int it, const BicgVecs& w, double* part, doub
   hipLaunchKernelGGL(mdot_partial_kernel, dim3(nb, 1), dim3(kDotThreads), 0, s, n, rpb, w.s, n, w.s, part + nb,
                      skip);
   hipLaunchKernelGGL(bicg_snorm_kernel, dim3(1), dim3(64), 0, s, it, nb, static_cast<const double*>(part + nb), tol,
-                     bnorm, c);
+                     c);
   hipLaunchKernelGGL(bicg_early_kernel, dim3(vb), dim3(256), 0, s, n, it, w.p, w.x, c.head);
   return hipGetLastError();
 }
 
-hipError_t bicg_after_t(int64_t n, const BicgVecs& w, double* part, double tol, double bnorm, const BicgCtl& c,
-                        hipStream_t s) {
+hipError_t bicg_after_t(int64_t n, const BicgVecs& w, double* part, double tol, const BicgCtl& c, hipStream_t s) {
   if (n <= kOneGroupRows) {
-    hipLaunchKernelGGL(bicg_t_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), w, tol, bnorm, c);
+    hipLaunchKernelGGL(bicg_t_one_kernel, dim3(1), dim3(kOneGroup), 0, s, static_cast<int>(n), w, tol, c);
     return hipGetLastError();
   }
   const int nb = mdot_blocks(n);
@@ -1560,7 +1711,7 @@ hipError_t bicg_after_t(int64_t n, const BicgVecs& w, double* part, double tol, 
   hipLaunchKernelGGL(mdot_partial_kernel, dim3(nb, 2), dim3(kDotThreads), 0, s, n, rpb, w.r, n, w.r, part + 4 * nb,
                      skip);
   hipLaunchKernelGGL(bicg_end_kernel, dim3(1), dim3(64), 0, s, nb, static_cast<const double*>(part + 4 * nb), tol,
-                     bnorm, c);
+                     c);
   hipLaunchKernelGGL(bicg_p_kernel, dim3(vb), dim3(256), 0, s, n, w.r, w.v, w.p, c.head);
   return hipGetLastError();
 }
