@@ -890,13 +890,13 @@ hipError_t launch_assemble_columns(int N, int NQI, bool analytical, int M, int64
 
 template <int N, int NQI, bool AN>
 static hipError_t launch_theta_t(int M, int64_t Lp, const double* pos, const double* ori, float* T, double* bpart,
-                                 float* Tv, double* cpart, const double* x0, double* apart, const PhysConsts& pc,
-                                 hipStream_t s, int* groups, _Float16* T16, float* S16) {
+                                 float* Tv, double* cpart, const double* x0, double* apart, bool far,
+                                 const PhysConsts& pc, hipStream_t s, int* groups, _Float16* T16, float* S16) {
   constexpr int PAIRS = kPairThreads / (3 * NQI);
   const PairGrid g = theta_grid(M, PAIRS);
   *groups = g.groups;
-  const bool all = M < far_min_fibers(AN);
-  if (!all) {
+  const bool all = !far;
+  if (far) {
     *groups += far_grid(M).groups;
     const hipError_t e =
         launch_assemble_far(N, NQI, AN, M, Lp, pos, ori, T, bpart, g.groups, Tv, cpart, x0, apart, pc, s, T16, S16);
@@ -913,22 +913,22 @@ static hipError_t launch_theta_t(int M, int64_t Lp, const double* pos, const dou
 
 template <int N, int NQI>
 static hipError_t launch_theta_n(bool an, int M, int64_t Lp, const double* pos, const double* ori, float* T,
-                                 double* bpart, float* Tv, double* cpart, const double* x0, double* apart,
+                                 double* bpart, float* Tv, double* cpart, const double* x0, double* apart, bool far,
                                  const PhysConsts& pc, hipStream_t s, int* groups, _Float16* T16, float* S16) {
-  return an ? launch_theta_t<N, NQI, true>(M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, pc, s, groups, T16, S16)
-            : launch_theta_t<N, NQI, false>(M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, pc, s, groups, T16, S16);
+  return an ? launch_theta_t<N, NQI, true>(M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, far, pc, s, groups, T16, S16)
+            : launch_theta_t<N, NQI, false>(M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, far, pc, s, groups, T16, S16);
 }
 
 #define RF_TH_CASE(NN)                                                                             \
   case NN:                                                                                         \
-    if (NQI == 4) return launch_theta_n<NN, 4>(analytical, M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, pc, s, groups, T16, S16); \
-    if (NQI == 8) return launch_theta_n<NN, 8>(analytical, M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, pc, s, groups, T16, S16); \
-    if (NQI == 16) return launch_theta_n<NN, 16>(analytical, M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, pc, s, groups, T16, S16); \
+    if (NQI == 4) return launch_theta_n<NN, 4>(analytical, M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, far, pc, s, groups, T16, S16); \
+    if (NQI == 8) return launch_theta_n<NN, 8>(analytical, M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, far, pc, s, groups, T16, S16); \
+    if (NQI == 16) return launch_theta_n<NN, 16>(analytical, M, Lp, pos, ori, T, bpart, Tv, cpart, x0, apart, far, pc, s, groups, T16, S16); \
     return hipErrorInvalidValue;
 
 hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
                                  const double* ori, float* T, double* bpart, float* Tv, double* cpart,
-                                 const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, int* groups,
+                                 const double* x0, double* apart, bool far, const PhysConsts& pc, hipStream_t s, int* groups,
                                  _Float16* T16, float* S16) {
   switch (N) {
     RF_TH_CASE(1)

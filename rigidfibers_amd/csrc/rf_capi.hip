@@ -399,6 +399,16 @@ rf_status gmres_core(rf_simulation* s, const double* b, double* x, bool warm, do
   return RF_OK;
 }
 
+// Whether the theta form's assembly takes the far pairs from their nodes.  Not for
+// the direct solvers, whose solution carries the system's rounding undamped into
+// positions and orientations that are kept in FP64: every pair there keeps the
+// near kernel's, and costs them little (the assembly without and with the nodes
+// is 3.7 and 1.1 of 179 ms at M = 2000, 11.9 and 6.7 of 413 at M = 5000).
+bool far_pairs(const rf_simulation* s) {
+  return s->cfg.solver != RF_SOLVER_DIRECT && s->cfg.solver != RF_SOLVER_DIRECT_MIXED_BF16 &&
+         s->cfg.solver != RF_SOLVER_DIRECT_MIXED_FP16 && s->M >= rf::far_min_fibers(s->analytical);
+}
+
 // Initial guess of the iterative solvers in s->x, which holds the previous
 // solution x_n when there is one: PREVIOUS keeps it, EXTRAPOLATED replaces it
 // by 2 x_n - x_{n-1} once x_{n-1} is known and keeps x_n for the next solve.
@@ -985,8 +995,8 @@ rf_status rf_assemble_system(rf_simulation* s) {
       RF_TRY(assemble_operator(s, x0));
     else
       RF_HIP(rf::launch_assemble_theta(s->N, s->NQI, s->analytical, s->M, s->Lp, s->pos[s->cur], s->ori[s->cur], s->T,
-                                     s->bpart, s->Tv, s->cpart, x0, x0 ? s->apart : nullptr, s->pc, s->stream,
-                                     &s->bgroups, s->T16, s->S16));
+                                       s->bpart, s->Tv, s->cpart, x0, x0 ? s->apart : nullptr, far_pairs(s), s->pc,
+                                       s->stream, &s->bgroups, s->T16, s->S16));
     RF_HIP(hipEventRecord(s->ev[6], s->stream));
     s->tori = s->cur;
     s->tori_valid = true;

@@ -53,9 +53,11 @@ hipError_t launch_assemble_far(int N, int NQI, bool analytical, int M, int64_t L
                                const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, _Float16* T16,
                                float* S16);
 int64_t theta_stride(int M, int N);
+// far: the far pairs by assemble_far_kernel (from far_min_fibers fibers on).
 hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
                                  const double* ori, float* T, double* bpart, float* Tv, double* cpart,
-                                 const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, int* groups,
+                                 const double* x0, double* apart, bool far, const PhysConsts& pc, hipStream_t s,
+                                 int* groups,
                                  _Float16* T16 = nullptr, float* S16 = nullptr);
 // With x0, the theta assembly also writes each group's off-diagonal product
 // rows sum_{j in group} A_ij x0_j into apart[group len + row].  With T16 it
