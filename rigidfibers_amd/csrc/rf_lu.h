@@ -90,16 +90,12 @@ struct LuResult {
 // hold row block r / 32 of A times sa[r / 32] and column block c / 32 of B
 // times sb[c / 32] (powers of two), which the update divides out.
 int gemm_stage_k(LuMode mode);
-// max_workgroups > 0 (subtracting form): at most that many workgroups (rounded
+// max_workgroups > 0 (subtracting form, mixed modes): at most that many workgroups (rounded
 // down to a multiple of 8), each taking several tiles, so that the rest of the
 // CUs stay free for work on other streams.
 hipError_t gemm_packed(LuMode mode, bool store, int64_t m, int64_t n, int64_t K, const void* At, int64_t ldak,
                        const void* Bt, int64_t ldbk, float* C, int64_t ldc, hipStream_t s,
                        const float* sa = nullptr, const float* sb = nullptr, int max_workgroups = 0);
-hipError_t gemm_packed_sub(LuMode mode, int64_t m, int64_t n, int64_t K, const void* At, int64_t ldak,
-                           const void* Bt, int64_t ldbk, float* C, int64_t ldc, hipStream_t s,
-                           const float* sa = nullptr, const float* sb = nullptr, int max_workgroups = 0);
-
 hipError_t lu_workspace_create(LuMode mode, int64_t n, int64_t lda, LuWorkspace* ws);
 int64_t lu_workspace_bytes(const LuWorkspace& ws);
 void lu_workspace_destroy(LuWorkspace* ws);
