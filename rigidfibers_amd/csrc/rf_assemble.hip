@@ -279,10 +279,6 @@ __global__ __launch_bounds__(kPairThreads) void assemble_kernel(int M, int64_t l
 //   T[(i * NC + c) * Lp + j * N + k_j],  NC = 3 + 6(N-1),  Lp >= M*N,
 // c = b for Q0_b, c = 3 + 6(k_i-1) + s for Theta_{k_i}[s] (s = xx yy zz xy xz yz),
 // zero for j == i (the identity diagonal blocks are implicit).
-//
-// Workgroup = one target fiber i x 8 consecutive source fibers per iteration
-// (lane = (source, q_i)); phase 2 jobs (column b, source, mode) are ordered so
-// that 40 consecutive lanes write 40 consecutive floats of each component.
 
 // Velocity operator (when the velocities integrate like the system): the
 // reference's velocity sums (fortran/update_velocities.incl:29-86) are
@@ -295,11 +291,7 @@ __global__ __launch_bounds__(kPairThreads) void assemble_kernel(int M, int64_t l
 // and in cpart[group][i][6] the constant sums of Phi0_{ij,0} F/2 and
 // Theta_{ij,0,P0} F/2 over its sources.
 
-// Column b of a symmetric 3x3 projection (v_a = S[(a, b)]) into its component
-// arrays s = xx yy zz xy xz yz at stride Lp: b = 0 writes xx xy xz, b = 1 yy yz,
-// b = 2 zz, so the three column jobs together write each component once.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 // The near pairs of one workgroup: target fiber i, source group gy (the far
 // pairs, by far_class, are assemble_far_block's; with `all` every pair is near).  The workgroup scans its
@@ -379,8 +371,8 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
   if (serving != nullptr) x0 = serving->x0;
   uint32_t lp32 = static_cast<uint32_t>(Lp);
   auto is_near = [&](int j) {
+    if (all) return j < je;  // the self pair too, as zeros: the sweeps stay aligned
     if (j >= je || j == i) return false;
-    if (all) return true;
     const double t0 = ori[3 * j], t1 = ori[3 * j + 1], t2 = ori[3 * j + 2];
     const int c = far_class(rule, xi[0] - pos[3 * j], xi[1] - pos[3 * j + 1], xi[2] - pos[3 * j + 2], ti2,
                             fma(t2, t2, fma(t1, t1, t0 * t0)));
@@ -427,7 +419,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       modes[kMaxTerms + t] = pc.eigen[t];
     }
   // the self pair
-  if (!SEGMENTS && i >= jb && i < je) {
+  if (!SEGMENTS && !all && i >= jb && i < je) {
     const uint32_t col = static_cast<uint32_t>(i) * N;
     for (int r = tid; r < NC * N; r += kPairThreads) {
       const uint32_t u = r / N, k = r - (r / N) * N;
@@ -470,10 +462,12 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       }
     pend += found;
     __syncthreads();
+    int head = 0;  // with `all`: from the front (a scan is a whole number of sweeps), in blocks of consecutive sources
     while (pend >= PAIRS || (last && pend > 0)) {
       const int take = min(pend, PAIRS);
       pend -= take;
-      const int* const js_ = nlist + pend;  // this sweep's sources
+      const int* const js_ = nlist + (all ? head : pend);  // this sweep's sources
+      head += take;
       // first column of source slot q
       auto col0 = [&](int q) { return SEGMENTS ? (formed + q) * N : js_[q] * N; };
       if constexpr (SEGMENTS) {
@@ -482,9 +476,10 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       if (tid < PAIRS) smax[tid] = 0u;
       if (p < take) {
         const int j = js_[p];
-        float acc[NM][6];
-        inner_integrals<N, NQI, ANALYTIC>(xi, tid_, ti, sq_d, sq, pos[3 * j], pos[3 * j + 1], pos[3 * j + 2],
-                                          ori[3 * j], ori[3 * j + 1], ori[3 * j + 2], pc, acc);
+        float acc[NM][6] = {};
+        if (j != i)
+          inner_integrals<N, NQI, ANALYTIC>(xi, tid_, ti, sq_d, sq, pos[3 * j], pos[3 * j + 1], pos[3 * j + 2],
+                                            ori[3 * j], ori[3 * j + 1], ori[3 * j + 2], pc, acc);
 #pragma unroll
         for (int m = 0; m < NM; ++m)
 #pragma unroll
@@ -533,7 +528,35 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
         const int c = (u - 3) - 6 * (kk - 2);
         return Pj[kk * RP + c * CB + PAIRS + pm];
       };
-      for (int job = tid; job < NC * PN; job += kPairThreads) {
+      // A whole sweep of consecutive sources is stored 16 bytes at a time.
+      const bool wide = !HALF && !SEGMENTS && all && take == PAIRS && ((js_[0] * N) & 3) == 0;
+      if (wide) {
+        constexpr int NV = PN / 4;
+        const uint32_t c0 = static_cast<uint32_t>(js_[0]) * N;
+        for (int job = tid; job < NC * NV; job += kPairThreads) {
+          const int u = job / NV, pm = 4 * (job - u * NV);
+          floatx4 val;
+          if (u < 3) {
+            const float* b1 = Pj + RP + PAIRS + pm;
+            const floatx4 vx = *reinterpret_cast<const floatx4*>(b1 + sym_index(0, u) * CB);
+            const floatx4 vy = *reinterpret_cast<const floatx4*>(b1 + sym_index(1, u) * CB);
+            const floatx4 vz = *reinterpret_cast<const floatx4*>(b1 + sym_index(2, u) * CB);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) val[e] = vx[e] * ti[0] + vy[e] * ti[1] + vz[e] * ti[2];
+          } else {
+            const int kk = 2 + (u - 3) / 6, c = (u - 3) - 6 * (kk - 2);
+            val = *reinterpret_cast<const floatx4*>(Pj + kk * RP + c * CB + PAIRS + pm);
+          }
+          *reinterpret_cast<floatx4*>(Ti + (static_cast<uint32_t>(u) * lp32 + c0 + pm)) = val;
+        }
+        if (Vi)
+          for (int job = tid; job < 12 * NV; job += kPairThreads) {
+            const int w = job / NV, pm = 4 * (job - w * NV), kk = w < 6 ? 1 : 0, c = w < 6 ? w : w - 6;
+            *reinterpret_cast<floatx4*>(Vi + (static_cast<uint32_t>(w) * lp32 + c0 + pm)) =
+                *reinterpret_cast<const floatx4*>(Pj + kk * RP + c * CB + PAIRS + pm);
+          }
+      }
+      for (int job = wide ? NC * PN : tid; job < NC * PN; job += kPairThreads) {
         const int u = job / PN, pm = job - u * PN, s = pm / N;
         if (s >= take) continue;
         const float val = sys_val(u, pm);
@@ -546,7 +569,7 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
         }
       }
       // velocity operator: Theta_0 (projection 1), then Phi_0 (projection 0)
-      if (Vi) {
+      if (Vi && !wide) {
         for (int job = tid; job < 12 * PN; job += kPairThreads) {
           const int w = job / PN, pm = job - w * PN, s = pm / N;
           if (s >= take) continue;
