@@ -53,6 +53,8 @@ __host__ __device__ constexpr double legendre_value(int f, double s) {
 // So the rounded weights reproduce the exact ones' functional of 1 (even m) or
 // of s (odd m): from the largest weight to the smallest, each takes up the
 // rounding of those before it, which moves no weight by more than an ulp or so.
+// For the far pairs' weights; the near pairs, a few sources each, keep the
+// products of the rounded tables, whose weights are each nearer to the exact ones.
 template <class Real, int H>
 __host__ __device__ constexpr void round_weights(const double (&exact)[H], const double (&s)[H], bool odd,
                                                  Real (&out)[H]) {
@@ -103,23 +105,6 @@ struct Quad {
         P[m][q] = static_cast<float>(legendre_value(m, sd[q]));
         W[m][q] = w[q] * P[m][q];
       }
-    // W[m][Q-1-q] = (-1)^m W[m][q].  Modes 0 and 1 keep the products of the
-    // rounded tables, which the pairwise velocities take.  b's error against FP64
-    // went from 1.7 - 3.5e-6 to 0.4 - 1.6e-6 of its largest entry with round_weights
-    // (operator form, M = 600 - 1000).
-    for (int m = 2; m <= N; ++m) {
-      double e[Q / 2] = {}, u[Q / 2] = {};
-      float r[Q / 2] = {};
-      for (int q = 0; q < Q / 2; ++q) {
-        u[q] = sd[q];
-        e[q] = gw[q % 3] / NQI * legendre_value(m, sd[q]);
-      }
-      round_weights<float, Q / 2>(e, u, m & 1, r);
-      for (int q = 0; q < Q / 2; ++q) {
-        W[m][q] = r[q];
-        W[m][Q - 1 - q] = (m & 1) ? -r[q] : r[q];
-      }
-    }
   }
 };
 
