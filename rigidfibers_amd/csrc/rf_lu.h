@@ -17,20 +17,15 @@ enum class LuMode { kFP32, kBF16, kFP16 };
 constexpr int kLuNb = 64;       // diagonal block: pivoting happens inside it
 constexpr int kLuPanel = 1024;  // outer panel
 // Panels per trailing update (its K = kLuGroup kLuPanel).  Measured at
-// n = 75 000 in one run (BF16 / FP16 ms per step, trailing GEMM TFLOP/s):
-// 2 -> 495 / 456 (749 / 833), 3 -> 494 / 457 (787 / 878), 4 -> 508 / 470
-// (799 / 902: the longer in-group chains on the look-ahead stream cost more
-// than the faster update saves).
+// n = 75 000 (BF16 ms per solve): 2 -> 528, 3 -> 404, 4 -> 405 (K = 4096; 3 takes
+// less memory); at n = 30 000 in FP32 1 -> 170, 2 -> 170, 3 -> 174.
 constexpr int kLuGroup = 3;
 // The trailing update beside the look-ahead's panels (BF16 / FP16), once at
 // most kLuTailRows rows remain (where the panels' chain is the longer of the two):
 // kLuTailWorkgroups workgroups (one per CU) take its tiles, the other CUs run
 // the chain's small kernels as they come instead of waiting for a tile to end.
-// Measured at n = 75 000 (BF16 / FP16 ms per step, interleaved runs on two
-// boxes, against 448.6 / 409.5 and 455.7 / 414.0 without): 24 576 rows, 224
-// workgroups -2 / -2; 36 864, 224: -4 / -4.5; 49 152, 224: -4.4 / -2.9;
-// 36 864, 192: -8.1 / -7.8 and -8.5 / -8.7; 36 864, 160: -8.0 / -6.5;
-// 49 152, 192: -2.8 / -1.5.
+// BF16 ms per solve at n = 75 000: without 410.8; 36 864 rows, 192 workgroups
+// 404.2; 224 workgroups 407.6; 24 576 rows 408.0; 49 152 rows 407.1.
 constexpr int64_t kLuTailRows = 36864;
 constexpr int kLuTailWorkgroups = 192;
 
