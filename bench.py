@@ -14,29 +14,39 @@ run untimed, then exactly K steps are timed between two device
 synchronisations.  value = M * K / elapsed.
 
 Also reported:
-  roofline      the step's dominant kernel, the assembly (VALU-bound): its
-                algorithmic flops per launch / the mean duration of the
-                assembly kernel (HIP events around it on the library's
-                stream), against the peak for its FP64/FP32 mix at MI355X's
-                published 78.6 / 157.3 TFLOP/s (the time the flops take at
-                those rates).  Flops: numerical, 63 216 FP32 per ordered fiber
-                pair; analytical, per (pair, target node): 624 FP64 (moment
-                recurrences) + 400 FP32 (recombination) where the node lies
-                within the far-field radius of the source's centre, else 576
-                FP32 (8-point far-field rule: 8 kernel evaluations of 30 flop,
-                6 mirror sums and 36 FMAs per node pair), plus 7 920 FP32 per
-                pair for the projections; near and far nodes are counted on
-                the initial scene.  reference_algorithm_count
-                prices the reference's algorithm instead (FP64 recurrences for
-                every pair: 32 500 flop per ordered pair, 15 000 of them FP64)
-                against the same kernel time;
-  roofline_solver  iterative solvers: the solver's matvec (HBM-bound),
-                algorithmic bytes per launch (theta form: M * M * N * (3 +
-                6(N-1)) * 4, the FP32 numbers that define A; dense: n^2 * 4) /
-                mean launch duration, against 8 TB/s.  Direct solvers: the
-                LU's trailing-update GEMMs (MFMA-bound), their 2 m n K flops /
-                summed duration, against the dense MFMA peak of the mode (FP32
-                157.3, BF16/FP16 2500 TFLOP/s);
+  roofline      the step's dominant kernel.  Iterative solvers on the operator
+                form (large suspensions: the far pairs' kernel values are
+                formed in every product): that product, VALU-bound, 36 kernel
+                values per ordered pair of 48 FP32 flop each (30 for the
+                value, 18 for its products) / mean launch duration, against
+                FP32's published 157.3 TFLOP/s.  Iterative solvers otherwise:
+                the assembly, as roofline_assembly.  Direct solvers:
+                roofline_solver;
+  roofline_assembly  the assembly (VALU-bound): its algorithmic flops / the
+                mean duration of its launches (HIP events around them on the
+                library's stream), against the peak for its FP64/FP32 mix at
+                the published 78.6 / 157.3 TFLOP/s (the time the flops take
+                at those rates).  Flops per ordered pair: far, 36 or 64 kernel
+                values (by distance) of 48 flop (operator form, where only
+                their sums are formed) or 102 (stored: with the projections);
+                near, numerical: 63 216 FP32; near, analytical, per (pair,
+                target node): 624 FP64 (moment recurrences) + 400 FP32
+                (recombination) where the node lies within the far-field
+                radius of the source's centre, else 576 FP32 (8-point rule),
+                plus 7 920 FP32 per pair for the projections; counted on the
+                initial scene.  The dense form and the direct solvers take
+                every pair as near.  reference_algorithm_count prices the
+                reference's algorithm instead (FP64 recurrences for every
+                pair: 32 500 flop per ordered pair, 15 000 of them FP64)
+                against the same time;
+  roofline_solver  iterative solvers: the solver's matvec.  Operator form: as
+                roofline.  Stored forms (HBM-bound): algorithmic bytes per
+                launch (theta form: M * M * N * (3 + 6(N-1)) * 4, the FP32
+                numbers that define A; dense: n^2 * 4) / mean launch duration,
+                against 8 TB/s.  Direct solvers: the LU's trailing-update GEMMs
+                (MFMA-bound), their 2 m n K flops / summed duration, against
+                the dense MFMA peak of the mode (FP32 157.3, BF16/FP16 2500
+                TFLOP/s);
   precision     plain FP32 LU against the BF16- and FP16-MFMA LUs with FP64
                 refinement (to 1e-10) on the same scene: fiber-steps/s, the
                 speed-up, the relative position error against the FP32-LU run
@@ -47,8 +57,8 @@ Also reported:
                 number density against the oracle's trajectory;
   serving       the serving stream with continuous batching against the same
                 stream one request at a time: p50/p99 step and request latency;
-  large         M = 10 000: GMRES-IR on the FP16 theta copy against plain
-                GMRES on the FP32 theta system (speed-up, position difference);
+  large         M = 10 000: GMRES-IR against plain GMRES, both on the operator
+                form (speed-up, position difference);
   cpu_baseline  the FP32 OpenMP port of the reference Fortran (oracle build
                 librf_oracle32.so) on a bounded sample: the rows of S target
                 fibers assembled against all 5000 sources, their velocities,
@@ -72,8 +82,8 @@ HBM_PEAK_GBS = 8000.0
 # the main thread to one place
 CPUS_AVAILABLE = len(os.sched_getaffinity(0))
 MFMA_PEAK_TFLOPS = {"direct": 157.3, "mixed-bf16": 2500.0, "mixed-fp16": 2500.0}
-GEMM_KERNEL = {"direct": "gemm_packed_sub_kernel<float>", "mixed-bf16": "gemm_packed_sub_kernel<__bf16>",
-               "mixed-fp16": "gemm_packed_sub_kernel<_Float16>"}
+GEMM_KERNEL = {"direct": "gemm_packed_kernel<float>", "mixed-bf16": "gemm_packed_kernel<__bf16>",
+               "mixed-fp16": "gemm_packed_kernel<_Float16>"}
 ITERATIVE = ("gmres", "bicgstab", "gmres-ir")
 
 
@@ -144,7 +154,30 @@ def far_field_radius(N=5):
     return float(vals[N])
 
 
-def assembly_flops(integration, pos, ori, N=5, nqi=8):
+def far_radii(N):
+    """The far pairs' centre distances (fine quadrature), read from the device source."""
+    import re
+
+    with open(os.path.join(ROOT, "rigidfibers_amd", "csrc", "rf_device.h")) as fh:
+        src = fh.read()
+    rows = re.search(r"fine\[kMaxTerms \+ 1\]\[2\] = \{(.*?)\};", src, re.S).group(1)
+    pairs = re.findall(r"\{([\d.]+), ([\d.]+)\}", rows)
+    return float(pairs[N][0]), float(pairs[N][1])
+
+
+# FP32 flop of the operator product per ordered pair: 36 kernel values of 30
+# flop, 18 more for each one's product with the source's node vector.
+OPERATOR_PAIR_FLOP = 36 * 48.0
+
+
+def operator_form(args, solver, N=5):
+    """Whether the library forms the far pairs in each product (matrix_format
+    auto, an iterative solver and a theta form of at least 450 MB)."""
+    return (solver in ITERATIVE and args.matrix_format == "auto" and
+            4.0 * args.fibers ** 2 * N * (3 + 6 * (N - 1)) >= 450e6)
+
+
+def assembly_flops(args, solver, integration, pos, ori, N=5, nqi=8):
     """(FP64, FP32) algorithmic flops of one assembly of this scene and the
     number of near (pair, node) combinations (see the module docstring)."""
     import numpy as np
@@ -152,30 +185,43 @@ def assembly_flops(integration, pos, ori, N=5, nqi=8):
 
     M = pos.size // 3
     pairs = float(M) * (M - 1)
+    P, T = pos.reshape(M, 3), ori.reshape(M, 3)
+    tree = cKDTree(P)
+    far32, near_pairs = 0.0, pairs
+    stored_far = args.matrix_format != "dense" and M >= 448
+    if solver in ITERATIVE and stored_far:
+        r6, r8 = far_radii(N)
+        within6, within8 = (int(tree.query_ball_point(P, r=r, return_length=True).sum()) - M for r in (r6, r8))
+        operator = operator_form(args, solver, N)
+        # the operator's product takes its own six-node pairs; its eight-node ones are stored
+        far32 = (pairs - within6) * 36 * (48.0 if operator else 102.0) + (within6 - within8) * 64 * 102.0
+        near_pairs = float(within8)
     if integration == "numerical":
-        return 0.0, pairs * 63_216.0, 0
+        return 0.0, far32 + near_pairs * 63_216.0, 0
     g = np.sqrt(15.0) / 5.0
     h = 2.0 / nqi
     s = np.array([(2.0 * (-1.0 + iv * h) + h + gp * h) / 2.0 for iv in range(nqi) for gp in (-g, 0.0, g)])
-    P, T = pos.reshape(M, 3), ori.reshape(M, 3)
     X = (P[:, None, :] + s[None, :, None] * T[:, None, :]).reshape(-1, 3)
     # source centres within the radius of each target node, less the node's own fiber
-    near = int(cKDTree(P).query_ball_point(X, r=far_field_radius(N), return_length=True).sum()) - M * s.size
-    far = pairs * s.size - near
-    return 624.0 * near, 400.0 * near + 576.0 * far + 7_920.0 * pairs, near
+    near = int(tree.query_ball_point(X, r=far_field_radius(N), return_length=True).sum()) - M * s.size
+    rule = max(near_pairs * s.size - near, 0.0)
+    return 624.0 * near, far32 + 400.0 * near + 576.0 * rule + 7_920.0 * near_pairs, near
 
 
 def step_bound(args, g):
     """The step at its bounds: the assembly's algorithmic flops at the
-    published FP64 / FP32 peaks, every matvec of the step and the stored
-    velocity pass at 8 TB/s."""
+    published FP64 / FP32 peaks, and every matvec of the step and the velocity
+    pass at the FP32 peak (operator form) or at 8 TB/s (stored forms)."""
     if not (args.solver == "gmres" and g["theta"]):
         return None
     M, N, K = args.fibers, 5, g["steps"]
     f64, f32, _ = g["asm_flops"]
     asm_ms = 1e3 * (f64 / (FP64_PEAK_TFLOPS * 1e12) + f32 / (FP32_PEAK_TFLOPS * 1e12))
-    mv_ms = 1e3 * M * (3 + 6 * (N - 1)) * M * N * 4.0 / (HBM_PEAK_GBS * 1e9)
-    vel_ms = 1e3 * M * 12 * M * N * 4.0 / (HBM_PEAK_GBS * 1e9)
+    if operator_form(args, args.solver, N):
+        mv_ms = vel_ms = 1e3 * float(M) * (M - 1) * OPERATOR_PAIR_FLOP / (FP32_PEAK_TFLOPS * 1e12)
+    else:
+        mv_ms = 1e3 * M * (3 + 6 * (N - 1)) * M * N * 4.0 / (HBM_PEAK_GBS * 1e9)
+        vel_ms = 1e3 * M * 12 * M * N * 4.0 / (HBM_PEAK_GBS * 1e9)
     matvecs = g["acc"]["gemv_launches"] / K
     total = asm_ms + matvecs * mv_ms + vel_ms
     return {"assembly_ms": round(asm_ms, 2), "matvec_ms": round(mv_ms, 3), "matvecs_per_step": round(matvecs, 2),
@@ -202,7 +248,7 @@ FP64_PEAK_TFLOPS, FP32_PEAK_TFLOPS = 78.6, 157.3
 
 
 def roofline_assembly(args, g):
-    """The assembly kernel against the time its algorithmic flops take at the
+    """The assembly's launches against the time its algorithmic flops take at the
     published FP64 / FP32 peaks."""
     M, K = args.fibers, g["steps"]
     f64, f32, near = g["asm_flops"]
@@ -212,8 +258,13 @@ def roofline_assembly(args, g):
     avg_ms = g["acc"]["assemble_kernel"] / K
     achieved = flop / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
     peak = flop / peak_s / 1e12
-    theta = g["theta"]
-    kernel = f"assemble_{'theta_' if theta else ''}kernel<5, 8, {'true' if args.integration == 'analytical' else 'false'}>"
+    an = "true" if args.integration == "analytical" else "false"
+    if operator_form(args, args.solver):
+        kernel = f"op_far_kernel<5> + assemble_segments_kernel<5, 8, {an}>"
+    elif g["theta"] and args.solver in ITERATIVE:
+        kernel = f"assemble_far_kernel<5> + assemble_near_kernel<5, 8, {an}>"
+    else:
+        kernel = f"assemble_{'near_' if g['theta'] else ''}kernel<5, 8, {an}>"
     # the reference algorithm's count (FP64 moment recurrences for every pair):
     # 32 500 flop per ordered pair, 15 000 of them FP64
     ref64, ref32 = 15_000.0 * pairs, 17_500.0 * pairs
@@ -225,7 +276,7 @@ def roofline_assembly(args, g):
     return {"bound": "valu", "kernel": kernel, "achieved": round(achieved, 2), "peak": round(peak, 2),
             "unit": "TFLOP/s", "frac": round(achieved / peak, 4) if peak > 0 else 0.0,
             "reference_algorithm_count": ref,
-            "traffic": measured_traffic(kernel.split("<")[0], M, 5) if theta else None,
+            "traffic": None,
             "flop_per_launch": flop, "fp64_flop_per_launch": f64, "fp32_flop_per_launch": f32,
             "near_pair_nodes": near, "pair_nodes": pairs * 24,
             "time_at_peak_ms": round(1e3 * peak_s, 3), "avg_launch_ms": round(avg_ms, 4)}
@@ -236,6 +287,13 @@ def roofline(args, solver, g):
     acc = g["acc"]
     if solver in ITERATIVE:
         theta = args.matrix_format == "theta" or args.matrix_format == "auto"
+        if operator_form(args, solver, N):
+            flop = float(M) * (M - 1) * OPERATOR_PAIR_FLOP
+            avg_ms = acc["gemv"] / max(acc["gemv_launches"], 1)
+            achieved = flop / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
+            return {"bound": "valu", "kernel": "op_far_kernel<5, false>", "achieved": round(achieved, 2),
+                    "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / FP32_PEAK_TFLOPS, 4),
+                    "traffic": None, "flop_per_launch": flop, "avg_launch_ms": round(avg_ms, 4)}
         if theta:  # 3 + 6(N-1) FP32 numbers per (target, source, source mode)
             per_launch, kernel = float(M) * (3 + 6 * (N - 1)) * M * N * 4.0, "gemv_theta_kernel"
         else:      # n^2 FP32 entries
@@ -263,7 +321,8 @@ def rel_err(a, b):
 def precision_study(args, pos, ori, plain=None):
     """Plain FP32 LU vs the BF16/FP16-MFMA LUs with FP64 refinement, same scene
     and steps; and, beside the headline's plain FP32 GMRES run (`plain`),
-    GMRES-IR with its inner solves on the FP16 copy of the theta-form system
+    GMRES-IR, its inner solves on the FP16 copy of the theta-form system or, on the
+    operator form, on its product
     (same steps and tolerance)."""
     out, ref = {}, None
     check = oracle_check(args) if args.oracle_check else {}
@@ -386,8 +445,8 @@ def serving(args):
 
 def large_suspension(args):
     """M = 10 000 fibers in a cube of side 60 (n = 150 000), numerical
-    integrals, GMRES restart 30 to 1e-8, 5 steps: GMRES-IR on the FP16 theta
-    copy (FP32 residuals) against plain GMRES on the FP32 theta system."""
+    integrals, GMRES restart 30 to 1e-8, 5 steps: GMRES-IR against plain GMRES,
+    both on the operator form (GMRES-IR then runs no FP16 product)."""
     from rigidfibers_amd.config import Parameters
     from rigidfibers_amd.scenes import cube
     from rigidfibers_amd.simulation import Simulation
@@ -421,7 +480,6 @@ def large_suspension(args):
                  "ms_per_step": round(1e3 * elapsed / args.large_steps, 2),
                  "solve_ms_per_step": round(solve / args.large_steps, 2), "iterations_per_step": iters,
                  "fp32_matvecs": gemv_n, "fp32_matvec_ms": round(gemv / max(gemv_n, 1), 4),
-                 "fp32_matvec_GBps": round(per32 / (gemv / max(gemv_n, 1) * 1e-3) / 1e9, 1) if gemv_n else None,
                  "device_bytes": dev}
         if half_n:
             per16 = per32 / 2 + float(M) * M * 4
@@ -558,7 +616,7 @@ def main():
     os.environ.setdefault("OMP_PLACES", "cores")
     pos, ori = build_scene(args.fibers, args.radius, args.seed)
     g = run_gpu(args, pos, ori, args.solver, args.steps, args.warmup)
-    g["asm_flops"] = assembly_flops(args.integration, pos, ori)
+    g["asm_flops"] = assembly_flops(args, args.solver, args.integration, pos, ori)
     M, K = args.fibers, args.steps
     value = M * K / g["elapsed"]
     fmt = ("theta" if args.matrix_format in ("auto", "theta") else "dense") if args.solver in ITERATIVE else "dense"
@@ -586,11 +644,13 @@ def main():
         "solver": {"iterations_per_step": g["iters"], "last": g["stats"]},
         "device_bytes": g["device_bytes"],
     }
-    # the roofline of the step's dominant kernel: the assembly for the
-    # iterative solvers, the LU's trailing updates for the direct ones
+    # the roofline of the step's dominant kernel: the product on the operator
+    # form, the assembly on the stored ones, the LU's trailing updates for the
+    # direct solvers
     asm = roofline_assembly(args, g)
     line["roofline_assembly"] = asm
-    line["roofline"] = asm if args.solver in ITERATIVE else line["roofline_solver"]
+    stored = args.solver in ITERATIVE and not operator_form(args, args.solver)
+    line["roofline"] = asm if stored else line["roofline_solver"]
     bound = step_bound(args, g)
     if bound is not None:
         line["step_bound"] = bound

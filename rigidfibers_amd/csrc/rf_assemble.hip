@@ -747,7 +747,7 @@ __global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(th
     const SusDev* __restrict__ sus, const int2* __restrict__ targets, PhysConsts pc) {
   const int2 e = targets[blockIdx.x];
   const SusDev& d = sus[e.x];
-  assemble_near_block<N, NQI, ANALYTIC>(e.y, 0, d.M, d.Lp, d.M < far_min_fibers(ANALYTIC), d.pos, d.ori, d.T, d.b, d.M, pc, d.Tv, d.cpart, nullptr,
+  assemble_near_block<N, NQI, ANALYTIC>(e.y, 0, d.M, d.Lp, d.M < kFarMinFibers, d.pos, d.ori, d.T, d.b, d.M, pc, d.Tv, d.cpart, nullptr,
                                          nullptr, nullptr, nullptr, &d);
 }
 

@@ -38,13 +38,16 @@ hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double
 // (Theta_0 and Phi0 of every source mode) and the velocity constants
 // cpart[group][i][6] (cpart then holds max_pair_groups(M) * M * 6 doubles).
 PairGrid theta_grid(int M, int sources_per_iteration);
-// Below this many fibers every pair takes the near kernel alone: the launch is
-// then its latency, and the far kernel's own (24 us at M = 100: a few wavefronts
-// with one batch after another) is longer than what it takes off the near one's.
-// Assembly in us, near alone / with the far kernel, at 0.1 fibers per unit
-// volume: numerical M = 200 78 / 84, 250 107 / 95, 400 187 / 126; analytical
-// 300 103 / 124, 400 140 / 131, 600 243 / 196.
-__host__ __device__ constexpr int far_min_fibers(bool analytical) { return analytical ? 384 : 240; }
+// Below this many fibers every pair takes the near kernel alone.  The launch is then
+// its latency, and the far kernel's own (24 us at M = 100: a few wavefronts with
+// one batch after another) is longer than what it takes off the near one's, or
+// saves little of a step: assembly in us, near alone / with the far kernel, at 0.1
+// fibers per unit volume: numerical M = 200 78 / 84, 250 107 / 95, 400 187 / 126;
+// analytical 300 103 / 124, 400 140 / 131, 600 243 / 196.  The line lies above the
+// sizes that are served in batches, so that a request of any of them is formed
+// the same way: trajectories through close contacts amplify the last bit of a
+// system a thousandfold and more.
+constexpr int kFarMinFibers = 448;
 // The far pairs (rf_far.hip): their sums go to the partial slots after the near
 // pairs' (slot0 on).
 PairGrid far_grid(int M);
@@ -53,7 +56,7 @@ hipError_t launch_assemble_far(int N, int NQI, bool analytical, int M, int64_t L
                                const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, _Float16* T16,
                                float* S16);
 int64_t theta_stride(int M, int N);
-// far: the far pairs by assemble_far_kernel (from far_min_fibers fibers on).
+// far: the far pairs by assemble_far_kernel (from kFarMinFibers fibers on).
 hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
                                  const double* ori, float* T, double* bpart, float* Tv, double* cpart,
                                  const double* x0, double* apart, bool far, const PhysConsts& pc, hipStream_t s,

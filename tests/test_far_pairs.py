@@ -99,10 +99,10 @@ def test_fewer_nodes_miss_the_bound():
     assert _error(5, 8, True, 6, near) > 1e-8
 
 
-CASES = [(5, 8, True, 385, 0.1, "gmres"), (5, 8, False, 257, 0.1, "gmres"), (5, 8, False, 300, 0.004, "gmres"),
-         (1, 8, False, 241, 0.05, "gmres"), (2, 16, False, 288, 0.1, "gmres"), (4, 4, True, 384, 0.02, "gmres"),
-         (6, 8, False, 250, 0.05, "gmres"), (7, 4, False, 263, 0.02, "gmres"), (8, 8, True, 400, 0.1, "gmres"),
-         (5, 8, True, 390, 0.05, "gmres-ir"), (8, 8, False, 240, 0.05, "gmres-ir")]
+CASES = [(5, 8, True, 449, 0.1, "gmres"), (5, 8, False, 457, 0.1, "gmres"), (5, 8, False, 460, 0.004, "gmres"),
+         (1, 8, False, 449, 0.05, "gmres"), (2, 16, False, 480, 0.1, "gmres"), (4, 4, True, 448, 0.02, "gmres"),
+         (6, 8, False, 450, 0.05, "gmres"), (7, 4, False, 463, 0.02, "gmres"), (8, 8, True, 448, 0.1, "gmres"),
+         (5, 8, True, 451, 0.05, "gmres-ir"), (8, 8, False, 448, 0.05, "gmres-ir")]
 
 
 @pytest.mark.gpu
