@@ -188,7 +188,7 @@ def assembly_flops(args, solver, integration, pos, ori, N=5, nqi=8):
     P, T = pos.reshape(M, 3), ori.reshape(M, 3)
     tree = cKDTree(P)
     far32, near_pairs = 0.0, pairs
-    stored_far = args.matrix_format != "dense" and M >= 448
+    stored_far = args.matrix_format != "dense" and M >= (448 if integration == "analytical" else 320)
     if solver in ITERATIVE and stored_far:
         r6, r8 = far_radii(N)
         within6, within8 = (int(tree.query_ball_point(P, r=r, return_length=True).sum()) - M for r in (r6, r8))

@@ -747,7 +747,7 @@ __global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(th
     const SusDev* __restrict__ sus, const int2* __restrict__ targets, PhysConsts pc) {
   const int2 e = targets[blockIdx.x];
   const SusDev& d = sus[e.x];
-  assemble_near_block<N, NQI, ANALYTIC>(e.y, 0, d.M, d.Lp, d.M < kFarMinFibers, d.pos, d.ori, d.T, d.b, d.M, pc, d.Tv, d.cpart, nullptr,
+  assemble_near_block<N, NQI, ANALYTIC>(e.y, 0, d.M, d.Lp, d.M < far_min_fibers(ANALYTIC), d.pos, d.ori, d.T, d.b, d.M, pc, d.Tv, d.cpart, nullptr,
                                          nullptr, nullptr, nullptr, &d);
 }
 
@@ -1157,10 +1157,12 @@ hipError_t launch_expand_theta(int N, int M, int64_t Lp, const float* T, const d
 }
 
 template <int N, int NQI>
-static hipError_t launch_theta_batch_n(bool an, int ntargets, const SusDev* sus, const int2* targets,
+static hipError_t launch_theta_batch_n(bool an, int ntargets, const SusDev* sus, const int2* targets, bool far,
                                        const PhysConsts& pc, hipStream_t s) {
-  const hipError_t e = launch_assemble_far_batch(N, NQI, an, ntargets, sus, targets, pc, s);
-  if (e != hipSuccess) return e;
+  if (far) {
+    const hipError_t e = launch_assemble_far_batch(N, NQI, an, ntargets, sus, targets, pc, s);
+    if (e != hipSuccess) return e;
+  }
   if (an)
     hipLaunchKernelGGL((assemble_near_batch_kernel<N, NQI, true>), dim3(ntargets), dim3(kPairThreads), 0, s, sus,
                        targets, pc);
@@ -1171,14 +1173,14 @@ static hipError_t launch_theta_batch_n(bool an, int ntargets, const SusDev* sus,
 }
 
 hipError_t launch_assemble_theta_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
-                                       const int2* targets, const PhysConsts& pc, hipStream_t s) {
+                                       const int2* targets, bool far, const PhysConsts& pc, hipStream_t s) {
   if (ntargets <= 0) return hipSuccess;
   switch (N) {
 #define RF_TB(NN)                                                                                 \
   case NN:                                                                                        \
-    if (NQI == 4) return launch_theta_batch_n<NN, 4>(analytical, ntargets, sus, targets, pc, s);   \
-    if (NQI == 8) return launch_theta_batch_n<NN, 8>(analytical, ntargets, sus, targets, pc, s);   \
-    if (NQI == 16) return launch_theta_batch_n<NN, 16>(analytical, ntargets, sus, targets, pc, s); \
+    if (NQI == 4) return launch_theta_batch_n<NN, 4>(analytical, ntargets, sus, targets, far, pc, s);   \
+    if (NQI == 8) return launch_theta_batch_n<NN, 8>(analytical, ntargets, sus, targets, far, pc, s);   \
+    if (NQI == 16) return launch_theta_batch_n<NN, 16>(analytical, ntargets, sus, targets, far, pc, s); \
     return hipErrorInvalidValue;
     RF_TB(1)
     RF_TB(2)

@@ -406,7 +406,7 @@ rf_status gmres_core(rf_simulation* s, const double* b, double* x, bool warm, do
 // is 3.7 and 1.1 of 179 ms at M = 2000, 11.9 and 6.7 of 413 at M = 5000).
 bool far_pairs(const rf_simulation* s) {
   return s->cfg.solver != RF_SOLVER_DIRECT && s->cfg.solver != RF_SOLVER_DIRECT_MIXED_BF16 &&
-         s->cfg.solver != RF_SOLVER_DIRECT_MIXED_FP16 && s->M >= rf::kFarMinFibers;
+         s->cfg.solver != RF_SOLVER_DIRECT_MIXED_FP16 && s->M >= rf::far_min_fibers(s->analytical);
 }
 
 // Initial guess of the iterative solvers in s->x, which holds the previous

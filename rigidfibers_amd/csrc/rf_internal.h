@@ -43,11 +43,12 @@ PairGrid theta_grid(int M, int sources_per_iteration);
 // one batch after another) is longer than what it takes off the near one's, or
 // saves little of a step: assembly in us, near alone / with the far kernel, at 0.1
 // fibers per unit volume: numerical M = 200 78 / 84, 250 107 / 95, 400 187 / 126;
-// analytical 300 103 / 124, 400 140 / 131, 600 243 / 196.  The line lies above the
-// sizes that are served in batches, so that a request of any of them is formed
-// the same way: trajectories through close contacts amplify the last bit of a
-// system a thousandfold and more.
-constexpr int kFarMinFibers = 448;
+// analytical 300 103 / 124, 400 140 / 131, 600 243 / 196.  The lines lie above the
+// first gains: small suspensions are formed one way, bit for bit, since
+// trajectories through close contacts amplify the last bit of a system a
+// thousandfold and more.  A batch of 24 suspensions of 16 to 400 fibers (numerical)
+// takes 37.0 ms with no far pairs, 36.5 with those from 320 and 33.9 from 240.
+__host__ __device__ constexpr int far_min_fibers(bool analytical) { return analytical ? 448 : 320; }
 // The far pairs (rf_far.hip): their sums go to the partial slots after the near
 // pairs' (slot0 on).
 PairGrid far_grid(int M);
@@ -56,7 +57,7 @@ hipError_t launch_assemble_far(int N, int NQI, bool analytical, int M, int64_t L
                                const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, _Float16* T16,
                                float* S16);
 int64_t theta_stride(int M, int N);
-// far: the far pairs by assemble_far_kernel (from kFarMinFibers fibers on).
+// far: the far pairs by assemble_far_kernel (from far_min_fibers fibers on).
 hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
                                  const double* ori, float* T, double* bpart, float* Tv, double* cpart,
                                  const double* x0, double* apart, bool far, const PhysConsts& pc, hipStream_t s,
@@ -228,8 +229,9 @@ hipError_t launch_orth_dots_batch(int nvb, int kdim, int phase, const SusDev* su
 
 hipError_t launch_assemble_far_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
                                      const int2* targets, const PhysConsts& pc, hipStream_t s);
+// far: one of the suspensions has far_min_fibers or more.
 hipError_t launch_assemble_theta_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
-                                       const int2* targets, const PhysConsts& pc, hipStream_t s);
+                                       const int2* targets, bool far, const PhysConsts& pc, hipStream_t s);
 hipError_t launch_gemv_theta_batch(int N, int ntargets, const SusDev* sus, const SusIter* it, const int2* targets,
                                    const PhysConsts& pc, hipStream_t s);
 hipError_t launch_velocities_stored_batch(int N, int ntargets, const SusDev* sus, const int2* targets,

@@ -451,8 +451,10 @@ bool solve_lockstep(rf_server* S) {
 bool tick(rf_server* S) {
   hipStream_t st = S->stream;
   if (!build_tables(S)) return false;
-  if (rf::launch_assemble_theta_batch(S->N, S->NQI, S->analytical, S->ntargets, S->d_sus, S->d_targets, S->pc, st) !=
-      hipSuccess)
+  const bool far = std::any_of(S->active.begin(), S->active.end(),
+                               [S](const auto* s) { return s->M >= rf::far_min_fibers(S->analytical); });
+  if (rf::launch_assemble_theta_batch(S->N, S->NQI, S->analytical, S->ntargets, S->d_sus, S->d_targets, far, S->pc,
+                                      st) != hipSuccess)
     return false;
   if (!solve_lockstep(S)) return false;
   if (rf::launch_velocities_stored_batch(S->N, S->ntargets, S->d_sus, S->d_targets, S->pc, st) != hipSuccess)
