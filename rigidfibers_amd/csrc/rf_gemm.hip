@@ -325,8 +325,8 @@ static void launch_tile(int64_t workgroups, int64_t m, int64_t n, int64_t K, con
 //          512 is nearly empty); 3000^2, 3072 452 / 536 / 706 (576); 12 000 x 1024,
 //          1024 211 / 212 / 257 (752); 6000^2, 3072 1665 / 1570 / 2115 (2209);
 //          24 576^2, 3072 25 677 / 24 919 / 25 101: 64 below 704 tiles of 128,
-//          else 128 (the matrix cores take four times as long for the same bytes
-//          as below: 256 has nothing to give);
+//          256 from 16 384 tiles of 256 (32 768^2), where the panels outgrow the
+//          MALL (the LU at n = 75 000: 2207 ms with 128, 2115 with 256), else 128;
 //   BF16   476^2, 1024 10 / 15 / 36; 1976 x 1024, 1024 11.0 / 12.6 / 27 (128 tiles
 //          of 128); 3976 x 1024, 1024 17.2 / 15.3 / 27.5 (256); 72 000 x 1024, 1024
 //          227 / 162 / 186; 27 000 x 1024, 2048 188 / 140 / 164; 6000^2, 3072 354 /
@@ -352,6 +352,8 @@ static void launch_gemm(bool store, int64_t m, int64_t n, int64_t K, const void*
   if constexpr (std::is_same<T, float>::value) {
     if (t128 < 704)
       go(Tile64{});
+    else if (tiles_of(m, n, 256) >= 16384)
+      go(std::integral_constant<int, 256>{});
     else
       go(Tile128{});
   } else {
