@@ -202,7 +202,10 @@ RF_API rf_status rf_step(rf_simulation* sim, int64_t current_timestep);
 
 /* The four phases of Simulation::step, for VALIDATE-style dumps between them. */
 RF_API rf_status rf_assemble_system(rf_simulation* sim);   /* assembleSystem, :331-399 */
-RF_API rf_status rf_solve_system(rf_simulation* sim);      /* solveSystem, :401-445 */
+/* solveSystem, :401-445.  RF_ERR_INVALID_ARGUMENT, with nothing launched, for
+ * a simulation that stores its near pairs only (RF_MATRIX_AUTO above) and has
+ * no system yet, or whose last assembly failed. */
+RF_API rf_status rf_solve_system(rf_simulation* sim);
 RF_API rf_status rf_update_velocities(rf_simulation* sim); /* updateVelocities, :447-489 */
 RF_API rf_status rf_update_fibers(rf_simulation* sim, int32_t first_timestep); /* updateFibers, :491-528 */
 RF_API rf_status rf_advance(rf_simulation* sim);           /* the buffer swaps, :307-311 */

@@ -31,6 +31,7 @@
 #include "rf_host.h"
 #include "rf_internal.h"
 #include "rf_lu.h"
+#include "rf_store.h"
 
 namespace {
 
@@ -56,6 +57,16 @@ rf_status fail(rf_status code, const std::string& msg) {
   } while (0)
 
 }  // namespace
+
+struct HipMemory {
+  static void* allocate(int64_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, static_cast<size_t>(bytes)) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  static void release(void* p) { (void)hipFree(p); }
+};
 
 struct rf_simulation {
   rf_config cfg{};
@@ -91,6 +102,7 @@ struct rf_simulation {
   int64_t Lp = 0;         // theta component stride
   bool oper = false;      // iterative solvers, large: products from the near pairs and the state (rf_operator.hip)
   rf::Operator op{};
+  rf::NearMemory<HipMemory> near_memory;  // op.near's
   unsigned long long* near_used = nullptr;  // op.near.used mirrored into pinned host memory
   hipEvent_t near_done = nullptr;
   int bgroups = 1;        // RHS partial slots written by the last assembly
@@ -142,7 +154,7 @@ struct rf_simulation {
   int ngemv = 0;
   hipEvent_t hev[2 * kGemvEvents] = {};  // the same for the FP16 products of GMRES-IR
   int nhalf = 0;
-  int64_t device_bytes = 0;
+  int64_t device_bytes = 0;  // without near_memory's
   std::vector<void*> allocations;
 
   template <typename T>
@@ -644,24 +656,14 @@ rf_status solve_direct(rf_simulation* s) {
   return RF_OK;
 }
 
-// Room for the operator's stored pairs: at least `floats`, in place of what
-// there is (which nothing in flight may use).
+// Room for the operator's stored pairs: `floats`, in place of what there is
+// (which nothing in flight may use).
 rf_status near_reserve(rf_simulation* s, int64_t floats) {
-  rf::NearStore& near = s->op.near;
-  if (near.data) (void)hipFree(near.data);
-  s->device_bytes -= near.capacity * static_cast<int64_t>(sizeof(float));
-  near.data = nullptr;
-  near.capacity = 0;
-  void* q = nullptr;
-  const hipError_t e = hipMalloc(&q, static_cast<size_t>(floats) * sizeof(float));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(RF_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(floats * 4) + " bytes for the near pairs failed: " +
-                                          hipGetErrorString(e));
-  }
-  near.data = static_cast<float*>(q);
-  near.capacity = floats;
-  s->device_bytes += floats * static_cast<int64_t>(sizeof(float));
+  const bool ok = s->near_memory.reserve(floats);
+  s->op.near.data = s->near_memory.data();
+  s->op.near.capacity = s->near_memory.capacity();
+  if (!ok)
+    return fail(RF_ERR_OUT_OF_MEMORY, "hipMalloc of " + std::to_string(floats * 4) + " bytes for the near pairs failed");
   return RF_OK;
 }
 
@@ -670,6 +672,10 @@ rf_status near_reserve(rf_simulation* s, int64_t floats) {
 // been counted: the launch that finds too little room says how much it needs,
 // the store grows by a quarter more than that and the launch is repeated.
 rf_status assemble_operator(rf_simulation* s, const double* x0) {
+  // the last system, its velocity operator and its dump end here
+  s->near_memory.begin();
+  s->vvalid = false;
+  s->tori_valid = false;
   double* const apart = x0 ? s->apart : nullptr;
   double* const cpart = s->vstored ? s->cpart : nullptr;
   for (int attempt = 0;; ++attempt) {
@@ -688,6 +694,7 @@ rf_status assemble_operator(rf_simulation* s, const double* x0) {
     RF_TRY(near_reserve(s, used + used / 4));
   }
   s->bgroups = 2;
+  s->near_memory.complete();
   return RF_OK;
 }
 
@@ -857,6 +864,11 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
     s->op.near.used = reinterpret_cast<unsigned long long*>(used);
     if (st == RF_OK) st = s->alloc(&s->op.near.base, static_cast<size_t>(M));
     if (st == RF_OK) st = s->alloc(&s->op.near.count, static_cast<size_t>(M));
+    // no pairs until an assembly has listed them
+    if (st == RF_OK &&
+        (hipMemsetAsync(s->op.near.base, 0, static_cast<size_t>(M) * sizeof(*s->op.near.base), s->stream) != hipSuccess ||
+         hipMemsetAsync(s->op.near.count, 0, static_cast<size_t>(M) * sizeof(*s->op.near.count), s->stream) != hipSuccess))
+      st = fail(RF_ERR_DEVICE, "hipMemsetAsync of the near pairs' counts failed");
     s->op.near.velocity = s->vstored ? 1 : 0;
     if (st == RF_OK) st = s->alloc(&s->op.nodes, rf::op_node_doubles(M, s->N));
     if (st == RF_OK) st = s->alloc(&s->op.part, rf::op_part_doubles(M, s->N));
@@ -963,7 +975,7 @@ void rf_destroy(rf_simulation* s) {
   if (s->stream) (void)hipStreamSynchronize(s->stream);
   rf::lu_workspace_destroy(&s->lu);
   for (void* p : s->allocations) (void)hipFree(p);
-  if (s->op.near.data) (void)hipFree(s->op.near.data);
+  s->near_memory.release();
   if (s->near_done) (void)hipEventDestroy(s->near_done);
   for (auto& e : s->ev)
     if (e) (void)hipEventDestroy(e);
@@ -1018,6 +1030,8 @@ rf_status rf_assemble_system(rf_simulation* s) {
 
 rf_status rf_solve_system(rf_simulation* s) {
   if (!s) return fail(RF_ERR_INVALID_ARGUMENT, "simulation is NULL");
+  if (s->oper && !s->near_memory.holds_system())
+    return fail(RF_ERR_INVALID_ARGUMENT, "rf_solve_system without a system (none assembled, or its assembly failed)");
   s->ngemv = 0;
   s->nhalf = 0;
   s->lu_last = rf::LuResult{};
@@ -1261,7 +1275,7 @@ rf_status rf_get_timings(rf_simulation* s, rf_timings* t) {
   return RF_OK;
 }
 
-int64_t rf_device_bytes(const rf_simulation* s) { return s ? s->device_bytes : 0; }
+int64_t rf_device_bytes(const rf_simulation* s) { return s ? s->device_bytes + s->near_memory.bytes() : 0; }
 
 const char* rf_last_error(void) { return g_last_error.c_str(); }
 

@@ -1,0 +1,49 @@
+"""The operator form's system and the calls around it (rf_operator.hip, rf_store.h):
+a solve takes its loop bounds and addresses from the near store, so one without a
+successful assembly is refused on the host."""
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+
+
+def test_near_memory_holds_a_system_only_after_a_whole_assembly(tmp_path):
+    exe = tmp_path / "near_memory"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I",
+                    os.path.join(ROOT, "rigidfibers_amd", "csrc"),
+                    os.path.join(HERE, "near_memory", "near_memory.cpp"), "-o", str(exe)], check=True)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=30)
+    assert out.returncode == 0, out.stdout
+
+
+def _sim(solver, M=1000, **kw):
+    from rigidfibers_amd.config import Parameters
+    from rigidfibers_amd.scenes import cube
+    from rigidfibers_amd.simulation import Simulation
+
+    pos, ori = cube(M, (M / 0.03) ** (1.0 / 3.0), min_dist=0.4, seed=M)
+    params = Parameters(NUMBER_OF_FIBERS=M, GMRES_TOLERANCE=1e-8, BICGSTAB_TOLERANCE=1e-8)
+    return pos, ori, Simulation(params, pos, ori, solver=solver, **kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("solver", ["gmres", "bicgstab", "gmres-ir"])
+def test_solve_without_a_system_is_refused(solver):
+    from rigidfibers_amd import _lib
+
+    pos, ori, sim = _sim(solver)
+    with sim:
+        for _ in range(2):
+            with pytest.raises(_lib.RfError) as err:
+                sim.solve_system()
+            assert err.value.code == _lib.RF_ERR_INVALID_ARGUMENT
+        assert sim.solver_stats()["iterations"] == 0  # nothing ran
+        sim.assemble_system()
+        sim.solve_system()
+        _, b, x = sim.system()
+        assert sim.solver_stats()["converged"] and np.isfinite(x).all() and b.any()
+        assert sim.step(0) == 0
