@@ -394,6 +394,10 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) cnt += ncount[0][w];
     lp32 = static_cast<uint32_t>(near_stride(cnt, N));
+    if (tid < 3) {
+      store->pos[3 * i + tid] = pos[3 * i + tid];
+      store->ori[3 * i + tid] = ori[3 * i + tid];
+    }
     if (tid == 0) {
       const int64_t size = near_ints(cnt) + static_cast<int64_t>(NC + (store->velocity ? 12 : 0)) * lp32;
       const int64_t at = static_cast<int64_t>(atomicAdd(store->used, static_cast<unsigned long long>(size)));

@@ -278,8 +278,8 @@ hipError_t sim_gemv(rf_simulation* s, const double* x, double* part, double* y, 
     ++s->ngemv;
   }
   if (s->oper)
-    return rf::op_product(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, x, y, b, mode,
-                          s->pc, s->stream, e0, e1, skip);
+    return rf::op_product(s->N, s->NQI, s->analytical, s->M, s->op, x, y, b, mode, s->pc, s->stream, e0, e1,
+                          skip);
   if (s->theta)
     return rf::gemv_theta(s->N, s->M, s->Lp, s->T, s->ori[s->cur], x, y, b, mode, s->pc, s->stream, e0, e1, skip);
   return rf::gemv(s->plan, s->A, x, part, y, b, mode, s->stream, e0, e1, skip);
@@ -551,8 +551,8 @@ rf_status solve_bicgstab(rf_simulation* s) {
   for (int k = 0; k < maxit; ++k) {
     if (k > 0) {  // a pending restart: r = b - A x (untimed), r0 = p = r, rho = ||r||^2
       if (s->oper)
-        RF_HIP(rf::op_product(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->x, r,
-                              s->b, 1, s->pc, s->stream, nullptr, nullptr, &s->bicg.head->no_restart));
+        RF_HIP(rf::op_product(s->N, s->NQI, s->analytical, s->M, s->op, s->x, r, s->b, 1, s->pc, s->stream,
+                              nullptr, nullptr, &s->bicg.head->no_restart));
       else if (s->theta)
         RF_HIP(rf::gemv_theta(s->N, s->M, s->Lp, s->T, s->ori[s->cur], s->x, r, s->b, 1, s->pc, s->stream,
                               nullptr, nullptr, &s->bicg.head->no_restart));
@@ -685,8 +685,8 @@ rf_status assemble_operator(rf_simulation* s, const double* x0) {
     RF_HIP(hipMemcpyAsync(s->near_used, s->op.near.used, sizeof(*s->near_used), hipMemcpyDeviceToHost, s->stream));
     RF_HIP(hipEventRecord(s->near_done, s->stream));
     if (attempt == 0)  // on the GPU while the host waits for the count
-      RF_HIP(rf::op_assemble_far(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->bpart,
-                                 cpart, x0, apart, s->pc, s->stream));
+      RF_HIP(rf::op_assemble_far(s->N, s->NQI, s->analytical, s->M, s->op, s->bpart, cpart, x0, apart, s->pc,
+                                 s->stream));
     RF_HIP(hipEventSynchronize(s->near_done));
     const int64_t used = static_cast<int64_t>(*static_cast<volatile unsigned long long*>(s->near_used));
     if (used <= s->op.near.capacity) break;
@@ -869,6 +869,8 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
         (hipMemsetAsync(s->op.near.base, 0, static_cast<size_t>(M) * sizeof(*s->op.near.base), s->stream) != hipSuccess ||
          hipMemsetAsync(s->op.near.count, 0, static_cast<size_t>(M) * sizeof(*s->op.near.count), s->stream) != hipSuccess))
       st = fail(RF_ERR_DEVICE, "hipMemsetAsync of the near pairs' counts failed");
+    if (st == RF_OK) st = s->alloc(&s->op.near.pos, fiber3);
+    if (st == RF_OK) st = s->alloc(&s->op.near.ori, fiber3);
     s->op.near.velocity = s->vstored ? 1 : 0;
     if (st == RF_OK) st = s->alloc(&s->op.nodes, rf::op_node_doubles(M, s->N));
     if (st == RF_OK) st = s->alloc(&s->op.part, rf::op_part_doubles(M, s->N));
@@ -1056,8 +1058,8 @@ rf_status rf_solve_system(rf_simulation* s) {
 rf_status rf_update_velocities(rf_simulation* s) {
   if (!s) return fail(RF_ERR_INVALID_ARGUMENT, "simulation is NULL");
   if (s->oper && s->vstored && s->vvalid)
-    RF_HIP(rf::op_velocities(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op, s->cpart, s->x,
-                             s->pc, s->tv[s->vcur], s->rv[s->vcur], s->stream));
+    RF_HIP(rf::op_velocities(s->N, s->NQI, s->analytical, s->M, s->op, s->cpart, s->x, s->pc, s->tv[s->vcur],
+                             s->rv[s->vcur], s->stream));
   else if (s->vstored && s->vvalid)
     RF_HIP(rf::launch_velocities_stored(s->N, s->M, s->Lp, s->Tv, s->cpart, s->bgroups, s->ori[s->cur], s->x, s->pc,
                                         s->tv[s->vcur], s->rv[s->vcur], s->stream));

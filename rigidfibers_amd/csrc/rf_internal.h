@@ -81,6 +81,8 @@ struct NearStore {
   int64_t* base;
   int* count;
   int velocity;               // the segments hold the velocity operator
+  double* pos;                // the state the segments belong to (3 M each): a product's far pairs
+  double* ori;                // are formed from it, whatever the caller's state has become
 };
 __host__ __device__ inline int near_ints(int count) { return (count + 15) / 16 * 16; }
 __host__ __device__ inline int64_t near_stride(int count, int N) {
@@ -111,18 +113,15 @@ size_t op_part_doubles(int M, int N);
 hipError_t launch_assemble_near(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
                                 const NearStore& near, double* bpart, double* cpart, const double* x0, double* apart,
                                 const PhysConsts& pc, hipStream_t s);
-// The far pairs' sums into slot 1.
-hipError_t op_assemble_far(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
-                           const Operator& op, double* bpart, double* cpart, const double* x0, double* apart,
-                           const PhysConsts& pc, hipStream_t s);
+// The far pairs' sums into slot 1, after launch_assemble_near, whose state they take.
+hipError_t op_assemble_far(int N, int NQI, bool analytical, int M, const Operator& op, double* bpart, double* cpart,
+                           const double* x0, double* apart, const PhysConsts& pc, hipStream_t s);
 // y = A x (mode 0) or y = b - A x (mode 1).
-hipError_t op_product(int N, int NQI, bool analytical, int M, const double* pos, const double* ori, const Operator& op,
-                      const double* x, double* y, const double* b, int mode, const PhysConsts& pc, hipStream_t s,
-                      hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr, const int* skip = nullptr);
+hipError_t op_product(int N, int NQI, bool analytical, int M, const Operator& op, const double* x, double* y,
+                      const double* b, int mode, const PhysConsts& pc, hipStream_t s, hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr, const int* skip = nullptr);
 // Velocities from the solution x; cpart's two slots as the assembly wrote them.
-hipError_t op_velocities(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
-                         const Operator& op, const double* cpart, const double* x, const PhysConsts& pc, double* tvel,
-                         double* rvel, hipStream_t s);
+hipError_t op_velocities(int N, int NQI, bool analytical, int M, const Operator& op, const double* cpart,
+                         const double* x, const PhysConsts& pc, double* tvel, double* rvel, hipStream_t s);
 // r = b - (x0 + sum_g apart[g]): the residual of x0 from those partials.
 hipError_t launch_residual_groups(int groups, int64_t len, const double* apart, const double* b, const double* x0,
                                   double* r, hipStream_t s);

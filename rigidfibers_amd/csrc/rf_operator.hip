@@ -452,12 +452,13 @@ size_t op_part_doubles(int M, int N) {
 }
 
 template <int N, int RHS>
-static hipError_t op_far(int NQI, bool analytical, int M, const double* pos, const double* ori, const Operator& op,
-                         const double* x0, const double* x1, const PhysConsts& pc, hipStream_t s, const int* skip) {
+static hipError_t op_far(int NQI, bool analytical, int M, const Operator& op, const double* x0, const double* x1,
+                         const PhysConsts& pc, hipStream_t s, const int* skip) {
   constexpr int NP = op_nodes<N>();
   const PairGrid g = op_grid(M);
   const int variant = op_variant(NQI, analytical);
   const dim3 nb((M * NP + 255) / 256);
+  const double *pos = op.near.pos, *ori = op.near.ori;
   double* n1 = op.nodes + 4 * static_cast<int64_t>(M) * NP;
   hipLaunchKernelGGL(op_nodes_kernel<N>, nb, dim3(256), 0, s, M, variant, ori, x0, pc, op.nodes, skip);
   if (RHS > 1)
@@ -468,14 +469,13 @@ static hipError_t op_far(int NQI, bool analytical, int M, const double* pos, con
 }
 
 template <int N>
-static hipError_t op_assemble_far_n(int NQI, bool analytical, int M, const double* pos, const double* ori,
-                                    const Operator& op, double* b, double* c, const double* x0, double* ax,
-                                    const PhysConsts& pc, hipStream_t s) {
-  const hipError_t e = x0 ? op_far<N, 2>(NQI, analytical, M, pos, ori, op, nullptr, x0, pc, s, nullptr)
-                          : op_far<N, 1>(NQI, analytical, M, pos, ori, op, nullptr, nullptr, pc, s, nullptr);
+static hipError_t op_assemble_far_n(int NQI, bool analytical, int M, const Operator& op, double* b,
+                                    double* c, const double* x0, double* ax, const PhysConsts& pc, hipStream_t s) {
+  const hipError_t e = x0 ? op_far<N, 2>(NQI, analytical, M, op, nullptr, x0, pc, s, nullptr)
+                          : op_far<N, 1>(NQI, analytical, M, op, nullptr, nullptr, pc, s, nullptr);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(op_assemble_rows_kernel<N>, dim3(M), dim3(64), 0, s, M, op_variant(NQI, analytical),
-                     op_grid(M).groups, x0 ? 2 : 1, op.part, ori, b, c, ax, pc);
+                     op_grid(M).groups, x0 ? 2 : 1, op.part, op.near.ori, b, c, ax, pc);
   return hipGetLastError();
 }
 
@@ -492,60 +492,55 @@ static hipError_t op_assemble_far_n(int NQI, bool analytical, int M, const doubl
     default: return hipErrorInvalidValue; \
   }
 
-hipError_t op_assemble_far(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
-                           const Operator& op, double* bpart, double* cpart, const double* x0, double* apart,
-                           const PhysConsts& pc, hipStream_t s) {
+hipError_t op_assemble_far(int N, int NQI, bool analytical, int M, const Operator& op, double* bpart, double* cpart,
+                           const double* x0, double* apart, const PhysConsts& pc, hipStream_t s) {
   const int64_t n = 3LL * N * M;
   double* c = cpart ? cpart + static_cast<int64_t>(M) * 6 : nullptr;
   double* ax = apart ? apart + n : nullptr;
-#define RF_CALL(NN) op_assemble_far_n<NN>(NQI, analytical, M, pos, ori, op, bpart + n, c, x0, ax, pc, s)
+#define RF_CALL(NN) op_assemble_far_n<NN>(NQI, analytical, M, op, bpart + n, c, x0, ax, pc, s)
   RF_OP_SIZES(RF_CALL)
 #undef RF_CALL
 }
 
 template <int N>
-static hipError_t op_product_n(int NQI, bool analytical, int M, const double* pos, const double* ori,
-                               const Operator& op, const double* x, double* y, const double* b, int mode,
-                               const PhysConsts& pc, hipStream_t s, const int* skip) {
-  const hipError_t e = op_far<N, 1>(NQI, analytical, M, pos, ori, op, x, nullptr, pc, s, skip);
+static hipError_t op_product_n(int NQI, bool analytical, int M, const Operator& op, const double* x, double* y,
+                               const double* b, int mode, const PhysConsts& pc, hipStream_t s, const int* skip) {
+  const hipError_t e = op_far<N, 1>(NQI, analytical, M, op, x, nullptr, pc, s, skip);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(op_rows_kernel<N>, dim3(M), dim3(kOpRowThreads), 0, s, M, op_variant(NQI, analytical),
-                     op_grid(M).groups, op.near, op.part, ori, x, y, b, mode, pc, skip);
+                     op_grid(M).groups, op.near, op.part, op.near.ori, x, y, b, mode, pc, skip);
   return hipGetLastError();
 }
 
-static hipError_t op_product_any(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
-                                 const Operator& op, const double* x, double* y, const double* b, int mode,
-                                 const PhysConsts& pc, hipStream_t s, const int* skip) {
-#define RF_CALL(NN) op_product_n<NN>(NQI, analytical, M, pos, ori, op, x, y, b, mode, pc, s, skip)
+static hipError_t op_product_any(int N, int NQI, bool analytical, int M, const Operator& op, const double* x,
+                                 double* y, const double* b, int mode, const PhysConsts& pc, hipStream_t s,
+                                 const int* skip) {
+#define RF_CALL(NN) op_product_n<NN>(NQI, analytical, M, op, x, y, b, mode, pc, s, skip)
   RF_OP_SIZES(RF_CALL)
 #undef RF_CALL
 }
 
-hipError_t op_product(int N, int NQI, bool analytical, int M, const double* pos, const double* ori, const Operator& op,
-                      const double* x, double* y, const double* b, int mode, const PhysConsts& pc, hipStream_t s,
-                      hipEvent_t ev_begin, hipEvent_t ev_end, const int* skip) {
+hipError_t op_product(int N, int NQI, bool analytical, int M, const Operator& op, const double* x, double* y,
+                      const double* b, int mode, const PhysConsts& pc, hipStream_t s, hipEvent_t ev_begin, hipEvent_t ev_end, const int* skip) {
   if (ev_begin) (void)hipEventRecord(ev_begin, s);
-  const hipError_t e = op_product_any(N, NQI, analytical, M, pos, ori, op, x, y, b, mode, pc, s, skip);
+  const hipError_t e = op_product_any(N, NQI, analytical, M, op, x, y, b, mode, pc, s, skip);
   if (ev_end) (void)hipEventRecord(ev_end, s);
   return e;
 }
 
 template <int N>
-static hipError_t op_velocities_n(int NQI, bool analytical, int M, const double* pos, const double* ori,
-                                  const Operator& op, const double* cpart, const double* x, const PhysConsts& pc,
-                                  double* tvel, double* rvel, hipStream_t s) {
-  const hipError_t e = op_far<N, 1>(NQI, analytical, M, pos, ori, op, x, nullptr, pc, s, nullptr);
+static hipError_t op_velocities_n(int NQI, bool analytical, int M, const Operator& op, const double* cpart,
+                                  const double* x, const PhysConsts& pc, double* tvel, double* rvel, hipStream_t s) {
+  const hipError_t e = op_far<N, 1>(NQI, analytical, M, op, x, nullptr, pc, s, nullptr);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(op_velocity_kernel<N>, dim3(M), dim3(kOpRowThreads), 0, s, M, op_variant(NQI, analytical),
-                     op_grid(M).groups, op.near, op.part, cpart, ori, x, pc, tvel, rvel);
+                     op_grid(M).groups, op.near, op.part, cpart, op.near.ori, x, pc, tvel, rvel);
   return hipGetLastError();
 }
 
-hipError_t op_velocities(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
-                         const Operator& op, const double* cpart, const double* x, const PhysConsts& pc, double* tvel,
-                         double* rvel, hipStream_t s) {
-#define RF_CALL(NN) op_velocities_n<NN>(NQI, analytical, M, pos, ori, op, cpart, x, pc, tvel, rvel, s)
+hipError_t op_velocities(int N, int NQI, bool analytical, int M, const Operator& op, const double* cpart,
+                         const double* x, const PhysConsts& pc, double* tvel, double* rvel, hipStream_t s) {
+#define RF_CALL(NN) op_velocities_n<NN>(NQI, analytical, M, op, cpart, x, pc, tvel, rvel, s)
   RF_OP_SIZES(RF_CALL)
 #undef RF_CALL
 }

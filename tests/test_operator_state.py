@@ -1,6 +1,7 @@
 """The operator form's system and the calls around it (rf_operator.hip, rf_store.h):
 a solve takes its loop bounds and addresses from the near store, so one without a
-successful assembly is refused on the host."""
+successful assembly is refused on the host; and the system is the assembled one,
+whatever becomes of the state before the solve."""
 import os
 import subprocess
 
@@ -47,3 +48,32 @@ def test_solve_without_a_system_is_refused(solver):
         _, b, x = sim.system()
         assert sim.solver_stats()["converged"] and np.isfinite(x).all() and b.any()
         assert sim.step(0) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("solver,integration", [("gmres", "numerical"), ("bicgstab", "analytical"),
+                                                ("gmres-ir", "numerical")])
+def test_the_state_moves_before_the_solve(solver, integration):
+    """A solve after rf_set_state or rf_advance is of the assembled system: the same
+    kernels on the same numbers from the same start (zero), so bit for bit."""
+    def solution(move):
+        pos, ori, sim = _sim(solver, integration=integration, initial_guess="zero")
+        with sim:
+            sim.assemble_system()
+            move(sim, pos, ori)
+            sim.solve_system()
+            return sim.system()[1:]
+
+    def overwrite(sim, pos, ori):
+        sim.set_state(1.01 * pos, ori[::-1].copy())
+
+    def advance(sim, pos, ori):
+        sim.solve_system()
+        sim.update_velocities()
+        sim.update_fibers(True)
+        sim.advance()
+
+    b, x = solution(lambda *_: None)
+    for move in (overwrite, advance):
+        b1, x1 = solution(move)
+        assert np.array_equal(b1, b) and np.array_equal(x1, x)
