@@ -59,6 +59,11 @@ rf_status fail(rf_status code, const std::string& msg) {
 }  // namespace
 
 struct HipMemory {
+  static int current_device() {
+    int d = -1;
+    return hipGetDevice(&d) == hipSuccess ? d : -1;
+  }
+  static bool make_current(int device) { return device >= 0 && hipSetDevice(device) == hipSuccess; }
   static void* allocate(int64_t bytes) {
     void* p = nullptr;
     if (hipMalloc(&p, static_cast<size_t>(bytes)) == hipSuccess) return p;
@@ -818,6 +823,7 @@ rf_status rf_create(const rf_config* cfg, const double* positions, const double*
                                                                         : cfg->velocity_integration == RF_VELOCITY_ANALYTICAL;
   make_consts(*cfg, &s->pc);
   if (hipGetDevice(&s->device) != hipSuccess) return cleanup(fail(RF_ERR_DEVICE, "no HIP device"));
+  s->near_memory.set_device(s->device);
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
     return cleanup(fail(RF_ERR_DEVICE, "hipStreamCreate failed"));
   // Timing events: no system-scope fence, which halves what a recorded event

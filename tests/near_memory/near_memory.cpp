@@ -16,10 +16,17 @@
 struct Model {
   static std::set<void*> live;
   static bool full;
+  static int device, placed;  // the thread's current GPU, and the last allocation's
+  static int current_device() { return device; }
+  static bool make_current(int d) {
+    device = d;
+    return d < 2;
+  }
   static void* allocate(long bytes) {
     if (full) return nullptr;
     CHECK(live.empty());  // the old store has been given back
     void* p = std::malloc(bytes);
+    placed = device;
     live.insert(p);
     return p;
   }
@@ -30,6 +37,7 @@ struct Model {
 };
 std::set<void*> Model::live;
 bool Model::full = false;
+int Model::device = 0, Model::placed = -1;
 
 int main() {
   {
@@ -53,6 +61,19 @@ int main() {
     CHECK(m.holds_system() && m.capacity() == 1000);
     // growing voids what was stored, also outside an assembly
     CHECK(m.reserve(2000) && !m.holds_system());
+  }
+  CHECK(Model::live.empty());
+  for (int own = 0; own < 2; ++own) {
+    // the store of GPU `own` grows in a thread whose current GPU is the other
+    rf::NearMemory<Model> m;
+    m.set_device(own);
+    for (int caller = 0; caller < 2; ++caller) {
+      Model::device = caller;
+      CHECK(m.reserve(10) && Model::placed == own && Model::device == caller);
+      Model::full = true;
+      CHECK(!m.reserve(20) && Model::device == caller);
+      Model::full = false;
+    }
   }
   CHECK(Model::live.empty());
   std::puts("ok");

@@ -13,6 +13,7 @@ ROOT = os.path.dirname(HERE)
 
 
 def test_near_memory_holds_a_system_only_after_a_whole_assembly(tmp_path):
+    """It holds a system only after a whole assembly, and grows on the simulation's GPU."""
     exe = tmp_path / "near_memory"
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I",
                     os.path.join(ROOT, "rigidfibers_amd", "csrc"),
