@@ -419,8 +419,8 @@ rf_status gmres_core(rf_simulation* s, const double* b, double* x, bool warm, do
 // Whether the theta form's assembly takes the far pairs from their nodes.  Not for
 // the direct solvers, whose solution carries the system's rounding undamped into
 // positions and orientations that are kept in FP64: every pair there keeps the
-// near kernel's, and costs them little (the assembly without and with the nodes
-// is 3.7 and 1.1 of 179 ms at M = 2000, 11.9 and 6.7 of 413 at M = 5000).
+// target nodes, and costs them little (the assembly without and with the nodes
+// is 3.7 and 1.1 of 179 ms at M = 2000, 12.0 and 6.7 of 413 at M = 5000).
 bool far_pairs(const rf_simulation* s) {
   return s->cfg.solver != RF_SOLVER_DIRECT && s->cfg.solver != RF_SOLVER_DIRECT_MIXED_BF16 &&
          s->cfg.solver != RF_SOLVER_DIRECT_MIXED_FP16 && s->M >= rf::far_min_fibers(s->analytical);

@@ -649,7 +649,6 @@ __global__ __launch_bounds__(kFarThreads, 2) void assemble_far_batch_kernel(cons
   constexpr int NC = 3 + 6 * (N - 1);
   const int2 e = targets[blockIdx.x];
   const SusDev& d = sus[e.x];
-  if (d.M < far_min_fibers(variant & 1)) return;  // its pairs are all the near kernel's
   const int i = e.y;
   FarOut out{d.T + static_cast<int64_t>(i) * NC * d.Lp, d.Tv + static_cast<int64_t>(i) * 12 * d.Lp, nullptr, nullptr,
              d.x0, static_cast<uint32_t>(d.Lp)};

@@ -38,7 +38,7 @@ hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double
 // (Theta_0 and Phi0 of every source mode) and the velocity constants
 // cpart[group][i][6] (cpart then holds max_pair_groups(M) * M * 6 doubles).
 PairGrid theta_grid(int M, int sources_per_iteration);
-// Below this many fibers every pair takes the near kernel alone.  The launch is then
+// Below this many fibers one kernel forms every pair.  The launch is then
 // its latency, and the far kernel's own (24 us at M = 100: a few wavefronts with
 // one batch after another) is longer than what it takes off the near one's, or
 // saves little of a step: assembly in us, near alone / with the far kernel, at 0.1
@@ -228,9 +228,9 @@ hipError_t launch_orth_dots_batch(int nvb, int kdim, int phase, const SusDev* su
 
 hipError_t launch_assemble_far_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
                                      const int2* targets, const PhysConsts& pc, hipStream_t s);
-// far: one of the suspensions has far_min_fibers or more.
-hipError_t launch_assemble_theta_batch(int N, int NQI, bool analytical, int ntargets, const SusDev* sus,
-                                       const int2* targets, bool far, const PhysConsts& pc, hipStream_t s);
+// The first nfar targets are those of the suspensions of far_min_fibers and more.
+hipError_t launch_assemble_theta_batch(int N, int NQI, bool analytical, int nfar, int ntargets, const SusDev* sus,
+                                       const int2* targets, const PhysConsts& pc, hipStream_t s);
 hipError_t launch_gemv_theta_batch(int N, int ntargets, const SusDev* sus, const SusIter* it, const int2* targets,
                                    const PhysConsts& pc, hipStream_t s);
 hipError_t launch_velocities_stored_batch(int N, int ntargets, const SusDev* sus, const int2* targets,

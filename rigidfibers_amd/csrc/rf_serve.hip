@@ -148,6 +148,7 @@ struct rf_server {
   double* d_part = nullptr;
   size_t c_dsus = 0, c_hsus = 0, c_dit = 0, c_hit = 0, c_dt = 0, c_ht = 0, c_dv = 0, c_hv = 0, c_df = 0, c_hf = 0,
          c_part = 0;
+  int nfar = 0;  // targets of the suspensions with a far kernel, the first ones of the table
   int ntargets = 0, nvb = 0, nfb = 0;
   rf::SusCtl* d_ctl = nullptr;
   rf::SusCtl* h_ctl = nullptr;
@@ -276,9 +277,17 @@ bool build_tables(rf_server* S) {
     d.pos_next = s->pos[s->next];
     d.ori_next = s->ori[s->next];
     d.first = s->have_history ? 0 : 1;
-    for (int i = 0; i < s->M; ++i) S->h_targets[ti++] = make_int2(q, i);
     for (int b = 0; b < d.vb_count; ++b) S->h_vblocks[vi++] = make_int2(q, b);
     for (int b = 0; b < (s->M + 255) / 256; ++b) S->h_fblocks[fi++] = make_int2(q, b);
+  }
+  // the suspensions whose far pairs have a kernel of their own come first
+  for (int small = 0; small < 2; ++small) {
+    for (int q = 0; q < ns; ++q) {
+      const int M = S->active[q]->M;
+      if ((M < rf::far_min_fibers(S->analytical)) != (small == 1)) continue;
+      for (int i = 0; i < M; ++i) S->h_targets[ti++] = make_int2(q, i);
+    }
+    if (small == 0) S->nfar = ti;
   }
   S->ntargets = nt;
   S->nvb = nv;
@@ -451,10 +460,8 @@ bool solve_lockstep(rf_server* S) {
 bool tick(rf_server* S) {
   hipStream_t st = S->stream;
   if (!build_tables(S)) return false;
-  const bool far = std::any_of(S->active.begin(), S->active.end(),
-                               [S](const auto* s) { return s->M >= rf::far_min_fibers(S->analytical); });
-  if (rf::launch_assemble_theta_batch(S->N, S->NQI, S->analytical, S->ntargets, S->d_sus, S->d_targets, far, S->pc,
-                                      st) != hipSuccess)
+  if (rf::launch_assemble_theta_batch(S->N, S->NQI, S->analytical, S->nfar, S->ntargets, S->d_sus, S->d_targets,
+                                      S->pc, st) != hipSuccess)
     return false;
   if (!solve_lockstep(S)) return false;
   if (rf::launch_velocities_stored_batch(S->N, S->ntargets, S->d_sus, S->d_targets, S->pc, st) != hipSuccess)
