@@ -1458,9 +1458,7 @@ hipError_t launch_assemble_near(int N, int NQI, bool analytical, int M, const do
     RF_SEG(NN, 16)   \
     break;
   switch (N) {
-    RF_SEG_N(1)
-    RF_SEG_N(2)
-    RF_SEG_N(3)
+    RF_SEG_N(3)  // operator_form is for N >= 3
     RF_SEG_N(4)
     RF_SEG_N(5)
     RF_SEG_N(6)

@@ -276,7 +276,7 @@ struct SolveMirror {
   int progress;
   int used;       // GMRES: Arnoldi steps of the cycle; BiCGStab: iterations
   int nonfinite;  // 1: a vector of the iteration, 2: the right-hand side, 3: the first residual
-  int start;      // how the solve's (or cycle's) start ended it: 1 zero right-hand side, 2 tolerance met
+  int start;      // GMRES: how the cycle's start ended it: 1 zero right-hand side, 2 tolerance met
   int converged;  // BiCGStab
   int prods;      // BiCGStab: products that ran
   int restarts;   // BiCGStab

@@ -1300,19 +1300,16 @@ __device__ __forceinline__ void bicg_start_control(double b2, double r2, double 
   h.res = sqrt(r2);
   h.rho = h.res * h.res;
   h.alpha = h.omega = h.beta = 0.0;
-  c.mirror->start = 0;
   if (!isfinite(h.bnorm)) {
     h.nonfinite = 2;
     bicg_end(c);
   } else if (h.bnorm == 0.0) {
-    c.mirror->start = 1;
     h.converged = 1;
     bicg_end(c);
   } else if (!isfinite(h.res)) {
     h.nonfinite = 3;
     bicg_end(c);
   } else if (h.res / h.bnorm <= tol) {
-    c.mirror->start = 2;
     h.converged = 1;
     bicg_end(c);
   }

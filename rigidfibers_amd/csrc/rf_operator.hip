@@ -479,10 +479,9 @@ static hipError_t op_assemble_far_n(int NQI, bool analytical, int M, const Opera
   return hipGetLastError();
 }
 
+// operator_form is for N >= 3
 #define RF_OP_SIZES(CALL)  \
   switch (N) {             \
-    case 1: return CALL(1); \
-    case 2: return CALL(2); \
     case 3: return CALL(3); \
     case 4: return CALL(4); \
     case 5: return CALL(5); \
