@@ -685,7 +685,7 @@ rf_status assemble_operator(rf_simulation* s, const double* x0) {
   double* const cpart = s->vstored ? s->cpart : nullptr;
   for (int attempt = 0;; ++attempt) {
     RF_HIP(rf::fill(1, 0.0, reinterpret_cast<double*>(s->op.near.used), s->stream));
-    RF_HIP(rf::launch_assemble_near(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op.near,
+    RF_HIP(rf::launch_assemble_segments(s->N, s->NQI, s->analytical, s->M, s->pos[s->cur], s->ori[s->cur], s->op.near,
                                     s->bpart, cpart, x0, apart, s->pc, s->stream));
     RF_HIP(hipMemcpyAsync(s->near_used, s->op.near.used, sizeof(*s->near_used), hipMemcpyDeviceToHost, s->stream));
     RF_HIP(hipEventRecord(s->near_done, s->stream));

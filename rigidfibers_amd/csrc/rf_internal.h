@@ -56,6 +56,11 @@ hipError_t launch_assemble_far(int N, int NQI, bool analytical, int M, int64_t L
                                const double* ori, float* T, double* bpart, int slot0, float* Tv, double* cpart,
                                const double* x0, double* apart, const PhysConsts& pc, hipStream_t s, _Float16* T16,
                                float* S16);
+// The near pairs beside them, on theta_grid's grid.
+hipError_t launch_assemble_near(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
+                                const double* ori, float* T, double* bpart, const PairGrid& g, float* Tv,
+                                double* cpart, const double* x0, double* apart, const PhysConsts& pc, hipStream_t s,
+                                _Float16* T16, float* S16);
 int64_t theta_stride(int M, int N);
 // far: the far pairs by assemble_far_kernel (from far_min_fibers fibers on).
 hipError_t launch_assemble_theta(int N, int NQI, bool analytical, int M, int64_t Lp, const double* pos,
@@ -110,10 +115,10 @@ size_t op_node_doubles(int M, int N);
 size_t op_part_doubles(int M, int N);
 // The near pairs' segments, and their sums as launch_assemble_theta writes
 // them, into slot 0 of bpart, cpart and apart.
-hipError_t launch_assemble_near(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
-                                const NearStore& near, double* bpart, double* cpart, const double* x0, double* apart,
-                                const PhysConsts& pc, hipStream_t s);
-// The far pairs' sums into slot 1, after launch_assemble_near, whose state they take.
+hipError_t launch_assemble_segments(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
+                                    const NearStore& near, double* bpart, double* cpart, const double* x0,
+                                    double* apart, const PhysConsts& pc, hipStream_t s);
+// The far pairs' sums into slot 1, after launch_assemble_segments, whose state they take.
 hipError_t op_assemble_far(int N, int NQI, bool analytical, int M, const Operator& op, double* bpart, double* cpart,
                            const double* x0, double* apart, const PhysConsts& pc, hipStream_t s);
 // y = A x (mode 0) or y = b - A x (mode 1).

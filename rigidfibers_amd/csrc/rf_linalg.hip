@@ -352,6 +352,42 @@ hipError_t fill(int64_t n, double value, double* y, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Sums of the assembly's partials, one slot per source group.
+__global__ void sum_groups_kernel(int groups, int64_t len, const double* __restrict__ part, double* __restrict__ out) {
+  const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (r >= len) return;
+  double s = 0.0;
+  for (int g = 0; g < groups; ++g) s += part[static_cast<int64_t>(g) * len + r];
+  out[r] = s;
+}
+
+__global__ void residual_groups_kernel(int groups, int64_t len, const double* __restrict__ apart,
+                                       const double* __restrict__ b, const double* __restrict__ x0,
+                                       double* __restrict__ r) {
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (k >= len) return;
+  double s = 0.0;
+  for (int g = 0; g < groups; ++g) s += apart[static_cast<int64_t>(g) * len + k];
+  r[k] = b[k] - (s + x0[k]);  // identity diagonal blocks
+}
+
+hipError_t launch_residual_groups(int groups, int64_t len, const double* apart, const double* b, const double* x0,
+                                  double* r, hipStream_t s) {
+  const int threads = 256;
+  const int64_t blocks = (len + threads - 1) / threads;
+  hipLaunchKernelGGL(residual_groups_kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), 0, s, groups, len,
+                     apart, b, x0, r);
+  return hipGetLastError();
+}
+
+hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double* out, hipStream_t s) {
+  const int threads = 256;
+  const int64_t blocks = (len + threads - 1) / threads;
+  hipLaunchKernelGGL(sum_groups_kernel, dim3(static_cast<unsigned>(blocks)), dim3(threads), 0, s, groups, len, part,
+                     out);
+  return hipGetLastError();
+}
+
 __global__ void nonfinite_kernel(int64_t n, const double* __restrict__ x, int* __restrict__ flag) {
   const int64_t r = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (r < n && !isfinite(x[r])) {

@@ -19,7 +19,7 @@
 //
 // Precision as in the stored form: kernel values in FP32 from centre
 // differences in FP64, everything they multiply and all sums in FP64.
-#include "rf_internal.h"
+#include "rf_near.h"
 
 namespace rf {
 
@@ -414,6 +414,51 @@ __global__ __launch_bounds__(kOpRowThreads) void op_velocity_kernel(int M, int v
     tvel[3 * i + a] = (0.5 / d) * ((d + 2.0) * F[a] + (d - 2.0) * tF * t[a] + Sv[a]);
     rvel[3 * i + a] = (1.5 / d) * (Sv[3 + a] - t[a] * tS);
   }
+}
+
+// The pairs of a large suspension that a product does not form again: workgroup
+// = target fiber, every source.
+template <int N, int NQI, bool ANALYTIC>
+__global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(
+    theta_min_waves<N, NQI, ANALYTIC>(kProductBytes<N, NQI> + kListBytes<N, NQI>), 8))) void assemble_segments_kernel(
+    int M, const double* __restrict__ pos, const double* __restrict__ ori, NearStore store,
+    double* __restrict__ bpart, PhysConsts pc, double* __restrict__ cpart, const double* __restrict__ x0,
+    double* __restrict__ apart) {
+  assemble_near_block<N, NQI, ANALYTIC, false, true>(blockIdx.x, 0, M, 0, pos, ori, nullptr, bpart, M, pc, nullptr,
+                                                     cpart, x0, apart, nullptr, nullptr, nullptr, &store);
+}
+
+hipError_t launch_assemble_segments(int N, int NQI, bool analytical, int M, const double* pos, const double* ori,
+                                    const NearStore& near, double* bpart, double* cpart, const double* x0,
+                                    double* apart, const PhysConsts& pc, hipStream_t s) {
+  const dim3 grid(M), block(kPairThreads);
+#define RF_SEG(NN, QQ)                                                                                              \
+  if (NQI == QQ) {                                                                                                  \
+    if (analytical)                                                                                                 \
+      hipLaunchKernelGGL((assemble_segments_kernel<NN, QQ, true>), grid, block, 0, s, M, pos, ori, near, bpart, pc,  \
+                         cpart, x0, apart);                                                                         \
+    else                                                                                                            \
+      hipLaunchKernelGGL((assemble_segments_kernel<NN, QQ, false>), grid, block, 0, s, M, pos, ori, near, bpart, pc, \
+                         cpart, x0, apart);                                                                         \
+    return hipGetLastError();                                                                                       \
+  }
+#define RF_SEG_N(NN) \
+  case NN:           \
+    RF_SEG(NN, 4)    \
+    RF_SEG(NN, 8)    \
+    RF_SEG(NN, 16)   \
+    break;
+  switch (N) {
+    RF_SEG_N(3)  // operator_form is for N >= 3
+    RF_SEG_N(4)
+    RF_SEG_N(5)
+    RF_SEG_N(6)
+    RF_SEG_N(7)
+    RF_SEG_N(8)
+  }
+#undef RF_SEG_N
+#undef RF_SEG
+  return hipErrorInvalidValue;
 }
 
 // Source groups: a workgroup is (64 targets, one group), four wavefronts on
