@@ -78,3 +78,37 @@ def test_the_state_moves_before_the_solve(solver, integration):
     for move in (overwrite, advance):
         b1, x1 = solution(move)
         assert np.array_equal(b1, b) and np.array_equal(x1, x)
+
+
+@pytest.mark.gpu
+def test_noalloc_dump_forms_the_same_columns():
+    """rf_get_system_noalloc forms the operator form's dense matrix 12 source fibers
+    at a time (8 terms: 12 x 24 columns of 13 512 rows fill the 16 MiB staging
+    buffer), the last range 11 of 563: bit for bit rf_get_system's, the diagonal
+    blocks the identity."""
+    import ctypes as C
+
+    from rigidfibers_amd import _lib
+    from rigidfibers_amd.config import Parameters
+    from rigidfibers_amd.scenes import cube
+    from rigidfibers_amd.simulation import Simulation
+
+    M, N = 563, 8
+    pos, ori = cube(M, (M / 0.05) ** (1.0 / 3.0), min_dist=0.4, seed=M)
+    params = Parameters(NUMBER_OF_FIBERS=M, NUMBER_OF_TERMS_IN_FORCE_EXPANSION=N)
+    with Simulation(params, pos, ori, integration="analytical") as sim:
+        theta_bytes = 4 * M * M * N * (3 + 6 * (N - 1))
+        assert sim.device_bytes() < theta_bytes  # the operator form
+        sim.step(0)  # the matrix belongs to the state before the step
+        A0, b0, x0 = sim.system(with_matrix=True)
+        A1 = np.full((sim.n, sim.n), np.nan, dtype=np.float32, order="F")
+        b1, x1 = np.full(sim.n, np.nan), np.full(sim.n, np.nan)
+        _lib.check(sim._lib.rf_get_system_noalloc(sim._h, A1.ctypes.data_as(C.POINTER(C.c_float)),
+                                                  b1.ctypes.data_as(C.POINTER(C.c_double)),
+                                                  x1.ctypes.data_as(C.POINTER(C.c_double))))
+    assert np.array_equal(A0, A1) and np.array_equal(b0, b1) and np.array_equal(x0, x1)
+    for j in (0, 11, 12, 551, 552, 562):  # ends of ranges
+        d = slice(24 * j, 24 * (j + 1))
+        assert np.array_equal(A0[d, d], np.eye(24, dtype=np.float32))
+    r = b0[:2400] - A0[:2400].astype(np.float64) @ x0
+    assert np.linalg.norm(r) <= 1e-4 * np.linalg.norm(b0)
