@@ -17,18 +17,21 @@ Also reported:
   roofline      the step's dominant kernel.  Iterative solvers on the operator
                 form (large suspensions: the far pairs' kernel values are
                 formed in every product): that product, VALU-bound, 36 kernel
-                values per ordered pair of 48 FP32 flop each (30 for the
-                value, 18 for its products) / mean launch duration, against
-                FP32's published 157.3 TFLOP/s.  Iterative solvers otherwise:
-                the assembly, as roofline_assembly.  Direct solvers:
-                roofline_solver;
+                values per ordered pair of 19 FP32 flop (the value) and 16
+                FP64 flop (its products) each / mean launch duration, against
+                the peak for that mix at the published 157.3 / 78.6 TFLOP/s
+                (the time the flops take at those rates).  Iterative solvers
+                otherwise: the assembly, as roofline_assembly.  Direct
+                solvers: roofline_solver;
   roofline_assembly  the assembly (VALU-bound): its algorithmic flops / the
                 mean duration of its launches (HIP events around them on the
                 library's stream), against the peak for its FP64/FP32 mix at
                 the published 78.6 / 157.3 TFLOP/s (the time the flops take
-                at those rates).  Flops per ordered pair: far, 36 or 64 kernel
-                values (by distance) of 48 flop (operator form, where only
-                their sums are formed) or 102 (stored: with the projections);
+                at those rates).  Flops per ordered pair: far, on the
+                operator form 36 kernel values of 19 FP32 and 32 FP64 flop
+                (their sums with two densities; the nearer pairs are stored,
+                by their target nodes), on the stored form 36 or 64 (by
+                distance) of 102 FP32 flop (with the projections);
                 near, numerical: 63 216 FP32; near, analytical, per (pair,
                 target node): 624 FP64 (moment recurrences) + 400 FP32
                 (recombination) where the node lies within the far-field
@@ -57,8 +60,10 @@ Also reported:
                 number density against the oracle's trajectory;
   serving       the serving stream with continuous batching against the same
                 stream one request at a time: p50/p99 step and request latency;
-  large         M = 10 000: GMRES-IR against plain GMRES, both on the operator
-                form (speed-up, position difference);
+  large         M = 10 000: GMRES-IR on the FP16 theta copy against plain
+                GMRES on the FP32 theta system (speed-up, position difference),
+                and plain GMRES on the operator form, which the library takes
+                by itself at this size;
   cpu_baseline  the FP32 OpenMP port of the reference Fortran (oracle build
                 librf_oracle32.so) on a bounded sample: the rows of S target
                 fibers assembled against all 5000 sources, their velocities,
@@ -93,7 +98,7 @@ def build_scene(M, radius, seed):
     return ball(M, radius, min_dist=0.4, seed=seed)
 
 
-def run_gpu(args, pos, ori, solver, steps, warmup, tag="", capture_last=False):
+def run_gpu(args, pos, ori, solver, steps, warmup, tag="", capture_last=False, matrix_format=None):
     """Runs warmup + steps timesteps; with capture_last also returns the state
     the last step assembled its system from and that step's solution."""
     from rigidfibers_amd.config import Parameters
@@ -103,7 +108,8 @@ def run_gpu(args, pos, ori, solver, steps, warmup, tag="", capture_last=False):
     params = Parameters(NUMBER_OF_FIBERS=M, TIMESTEP=0.1, SLENDERNESS=0.01, NUMBER_OF_TERMS_IN_FORCE_EXPANSION=5,
                         NUMBER_OF_QUADRATURE_INTERVALS=8, GMRES_RESTART=args.restart,
                         GMRES_MAX_ITERATIONS=1000, GMRES_TOLERANCE=args.tol, BICGSTAB_TOLERANCE=args.tol)
-    matrix_format = args.matrix_format if solver in ITERATIVE else "auto"
+    if matrix_format is None:
+        matrix_format = args.matrix_format if solver in ITERATIVE else "auto"
     sim = Simulation(params, pos, ori, solver=solver, integration=args.integration, matrix_format=matrix_format,
                      velocity_operator=args.velocity_operator, refinement_tolerance=1e-10,
                      initial_guess=args.initial_guess,
@@ -165,9 +171,14 @@ def far_radii(N):
     return float(pairs[N][0]), float(pairs[N][1])
 
 
-# FP32 flop of the operator product per ordered pair: 36 kernel values of 30
-# flop, 18 more for each one's product with the source's node vector.
-OPERATOR_PAIR_FLOP = 36 * 48.0
+# Flops of the operator product per ordered pair: 36 kernel values of 19 FP32
+# flop, and 16 FP64 flop for each one's product with the source's node vector.
+OPERATOR_PAIR_F32, OPERATOR_PAIR_F64 = 36 * 19.0, 36 * 16.0
+
+
+def peak_seconds(f64, f32):
+    """The time these flops take at the published FP64 and FP32 rates."""
+    return f64 / (FP64_PEAK_TFLOPS * 1e12) + f32 / (FP32_PEAK_TFLOPS * 1e12)
 
 
 def operator_form(args, solver, N=5):
@@ -175,6 +186,12 @@ def operator_form(args, solver, N=5):
     auto, an iterative solver and a theta form of at least 450 MB)."""
     return (solver in ITERATIVE and args.matrix_format == "auto" and
             4.0 * args.fibers ** 2 * N * (3 + 6 * (N - 1)) >= 450e6)
+
+
+def stored_far(args, solver):
+    """Whether the theta form's far pairs have a kernel of their own."""
+    return (solver in ITERATIVE and args.matrix_format != "dense" and
+            args.fibers >= (448 if args.integration == "analytical" else 320))
 
 
 def assembly_flops(args, solver, integration, pos, ori, N=5, nqi=8):
@@ -187,17 +204,18 @@ def assembly_flops(args, solver, integration, pos, ori, N=5, nqi=8):
     pairs = float(M) * (M - 1)
     P, T = pos.reshape(M, 3), ori.reshape(M, 3)
     tree = cKDTree(P)
-    far32, near_pairs = 0.0, pairs
-    stored_far = args.matrix_format != "dense" and M >= (448 if integration == "analytical" else 320)
-    if solver in ITERATIVE and stored_far:
+    far64, far32, near_pairs = 0.0, 0.0, pairs
+    if stored_far(args, solver):
         r6, r8 = far_radii(N)
         within6, within8 = (int(tree.query_ball_point(P, r=r, return_length=True).sum()) - M for r in (r6, r8))
-        operator = operator_form(args, solver, N)
-        # the operator's product takes its own six-node pairs; its eight-node ones are stored
-        far32 = (pairs - within6) * 36 * (48.0 if operator else 102.0) + (within6 - within8) * 64 * 102.0
-        near_pairs = float(within8)
+        if operator_form(args, solver, N):  # the pairs within the first radius are stored
+            far32, far64 = (pairs - within6) * OPERATOR_PAIR_F32, 2.0 * (pairs - within6) * OPERATOR_PAIR_F64
+            near_pairs = float(within6)
+        else:
+            far32 = ((pairs - within6) * 36 + (within6 - within8) * 64) * 102.0
+            near_pairs = float(within8)
     if integration == "numerical":
-        return 0.0, far32 + near_pairs * 63_216.0, 0
+        return far64, far32 + near_pairs * 63_216.0, 0
     g = np.sqrt(15.0) / 5.0
     h = 2.0 / nqi
     s = np.array([(2.0 * (-1.0 + iv * h) + h + gp * h) / 2.0 for iv in range(nqi) for gp in (-g, 0.0, g)])
@@ -205,20 +223,21 @@ def assembly_flops(args, solver, integration, pos, ori, N=5, nqi=8):
     # source centres within the radius of each target node, less the node's own fiber
     near = int(tree.query_ball_point(X, r=far_field_radius(N), return_length=True).sum()) - M * s.size
     rule = max(near_pairs * s.size - near, 0.0)
-    return 624.0 * near, far32 + 400.0 * near + 576.0 * rule + 7_920.0 * near_pairs, near
+    return far64 + 624.0 * near, far32 + 400.0 * near + 576.0 * rule + 7_920.0 * near_pairs, near
 
 
 def step_bound(args, g):
     """The step at its bounds: the assembly's algorithmic flops at the
     published FP64 / FP32 peaks, and every matvec of the step and the velocity
-    pass at the FP32 peak (operator form) or at 8 TB/s (stored forms)."""
+    pass at the published FP64 / FP32 peaks (operator form) or at 8 TB/s (stored
+    forms)."""
     if not (args.solver == "gmres" and g["theta"]):
         return None
     M, N, K = args.fibers, 5, g["steps"]
     f64, f32, _ = g["asm_flops"]
-    asm_ms = 1e3 * (f64 / (FP64_PEAK_TFLOPS * 1e12) + f32 / (FP32_PEAK_TFLOPS * 1e12))
+    asm_ms = 1e3 * peak_seconds(f64, f32)
     if operator_form(args, args.solver, N):
-        mv_ms = vel_ms = 1e3 * float(M) * (M - 1) * OPERATOR_PAIR_FLOP / (FP32_PEAK_TFLOPS * 1e12)
+        mv_ms = vel_ms = 1e3 * float(M) * (M - 1) * peak_seconds(OPERATOR_PAIR_F64, OPERATOR_PAIR_F32)
     else:
         mv_ms = 1e3 * M * (3 + 6 * (N - 1)) * M * N * 4.0 / (HBM_PEAK_GBS * 1e9)
         vel_ms = 1e3 * M * 12 * M * N * 4.0 / (HBM_PEAK_GBS * 1e9)
@@ -254,17 +273,19 @@ def roofline_assembly(args, g):
     f64, f32, near = g["asm_flops"]
     pairs = float(M) * (M - 1)
     flop = f64 + f32
-    peak_s = f64 / (FP64_PEAK_TFLOPS * 1e12) + f32 / (FP32_PEAK_TFLOPS * 1e12)
+    peak_s = peak_seconds(f64, f32)
     avg_ms = g["acc"]["assemble_kernel"] / K
     achieved = flop / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
     peak = flop / peak_s / 1e12
     an = "true" if args.integration == "analytical" else "false"
     if operator_form(args, args.solver):
-        kernel = f"op_far_kernel<5> + assemble_segments_kernel<5, 8, {an}>"
-    elif g["theta"] and args.solver in ITERATIVE:
-        kernel = f"assemble_far_kernel<5> + assemble_near_kernel<5, 8, {an}>"
+        kernel = f"op_far_kernel<5, 2> + assemble_segments_kernel<5, 8, {an}>"
+    elif g["theta"] and stored_far(args, args.solver):
+        kernel = f"assemble_far_kernel<5, false> + assemble_near_kernel<5, 8, {an}, false>"
+    elif args.matrix_format == "dense":
+        kernel = f"assemble_kernel<5, 8, {an}>"
     else:
-        kernel = f"assemble_{'near_' if g['theta'] else ''}kernel<5, 8, {an}>"
+        kernel = f"assemble_theta_kernel<5, 8, {an}, false>"
     # the reference algorithm's count (FP64 moment recurrences for every pair):
     # 32 500 flop per ordered pair, 15 000 of them FP64
     ref64, ref32 = 15_000.0 * pairs, 17_500.0 * pairs
@@ -288,12 +309,15 @@ def roofline(args, solver, g):
     if solver in ITERATIVE:
         theta = args.matrix_format == "theta" or args.matrix_format == "auto"
         if operator_form(args, solver, N):
-            flop = float(M) * (M - 1) * OPERATOR_PAIR_FLOP
+            f64, f32 = (float(M) * (M - 1) * f for f in (OPERATOR_PAIR_F64, OPERATOR_PAIR_F32))
+            peak = (f64 + f32) / peak_seconds(f64, f32) / 1e12
             avg_ms = acc["gemv"] / max(acc["gemv_launches"], 1)
-            achieved = flop / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
-            return {"bound": "valu", "kernel": "op_far_kernel<5, false>", "achieved": round(achieved, 2),
-                    "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": round(achieved / FP32_PEAK_TFLOPS, 4),
-                    "traffic": None, "flop_per_launch": flop, "avg_launch_ms": round(avg_ms, 4)}
+            achieved = (f64 + f32) / (avg_ms * 1e-3) / 1e12 if avg_ms > 0 else 0.0
+            return {"bound": "valu", "kernel": "op_far_kernel<5, 1>", "achieved": round(achieved, 2),
+                    "peak": round(peak, 2), "unit": "TFLOP/s", "frac": round(achieved / peak, 4),
+                    "traffic": None, "flop_per_launch": f64 + f32, "fp64_flop_per_launch": f64,
+                    "fp32_flop_per_launch": f32, "time_at_peak_ms": round(1e3 * peak_seconds(f64, f32), 4),
+                    "avg_launch_ms": round(avg_ms, 4)}
         if theta:  # 3 + 6(N-1) FP32 numbers per (target, source, source mode)
             per_launch, kernel = float(M) * (3 + 6 * (N - 1)) * M * N * 4.0, "gemv_theta_kernel"
         else:      # n^2 FP32 entries
@@ -321,9 +345,8 @@ def rel_err(a, b):
 def precision_study(args, pos, ori, plain=None):
     """Plain FP32 LU vs the BF16/FP16-MFMA LUs with FP64 refinement, same scene
     and steps; and, beside the headline's plain FP32 GMRES run (`plain`),
-    GMRES-IR, its inner solves on the FP16 copy of the theta-form system or, on the
-    operator form, on its product
-    (same steps and tolerance)."""
+    GMRES-IR with its inner solves on the FP16 copy of the theta-form system and
+    plain GMRES on that system (same steps and tolerance)."""
     out, ref = {}, None
     check = oracle_check(args) if args.oracle_check else {}
     for solver in ("direct", "mixed-bf16", "mixed-fp16"):
@@ -345,7 +368,10 @@ def precision_study(args, pos, ori, plain=None):
     out["steps"] = args.lu_steps
     out["warmup"] = 1
     if plain is not None:
-        g = run_gpu(args, pos, ori, "gmres-ir", args.steps, args.warmup, tag="precision ")
+        headline_rate = args.fibers * plain["steps"] / plain["elapsed"]
+        if operator_form(args, args.solver):
+            plain = run_gpu(args, pos, ori, "gmres", args.steps, args.warmup, tag="precision ", matrix_format="theta")
+        g = run_gpu(args, pos, ori, "gmres-ir", args.steps, args.warmup, tag="precision ", matrix_format="theta")
         rate = args.fibers * g["steps"] / g["elapsed"]
         plain_rate = args.fibers * plain["steps"] / plain["elapsed"]
         out["gmres_ir_fp16"] = {
@@ -354,6 +380,7 @@ def precision_study(args, pos, ori, plain=None):
             "plain_solve_ms_per_step": round(plain["phases"]["solve_system"] / plain["steps"], 2),
             "iterations_per_step": g["iters"], "steps": g["steps"],
             "speedup_vs_plain_fp32_gmres": round(rate / plain_rate, 3),
+            "speedup_vs_headline": round(rate / headline_rate, 3),
             "pos_rel_err_vs_plain_fp32_gmres": rel_err(g["pos"], plain["pos"]),
             "ori_rel_err_vs_plain_fp32_gmres": rel_err(g["ori"], plain["ori"])}
     return out
@@ -445,8 +472,9 @@ def serving(args):
 
 def large_suspension(args):
     """M = 10 000 fibers in a cube of side 60 (n = 150 000), numerical
-    integrals, GMRES restart 30 to 1e-8, 5 steps: GMRES-IR against plain GMRES,
-    both on the operator form (GMRES-IR then runs no FP16 product)."""
+    integrals, GMRES restart 30 to 1e-8, 5 steps: GMRES-IR on the FP16 theta
+    copy (FP32 residuals) against plain GMRES on the FP32 theta system, and plain
+    GMRES on the operator form ("auto")."""
     from rigidfibers_amd.config import Parameters
     from rigidfibers_amd.scenes import cube
     from rigidfibers_amd.simulation import Simulation
@@ -458,8 +486,9 @@ def large_suspension(args):
                         GMRES_TOLERANCE=1e-8)
     out, ref = {"workload": f"M={M} cube of side {60.0 * (M / 10000.0) ** (1.0 / 3.0):g}, numerical, GMRES(30) "
                             f"tol 1e-8, 1 warm-up + {args.large_steps} timed steps"}, None
-    for solver in ("gmres", "gmres-ir"):
-        with Simulation(params, pos, ori, solver=solver, integration="numerical") as sim:
+    for key, solver, fmt in (("gmres", "gmres", "theta"), ("gmres_ir", "gmres-ir", "theta"),
+                             ("gmres_operator", "gmres", "auto")):
+        with Simulation(params, pos, ori, solver=solver, integration="numerical", matrix_format=fmt) as sim:
             iters, gemv, gemv_n, half, half_n, solve = [], 0.0, 0, 0.0, 0, 0.0
             sim.step(0)  # untimed warm-up (cold GMRES start)
             t0 = time.perf_counter()
@@ -481,6 +510,8 @@ def large_suspension(args):
                  "solve_ms_per_step": round(solve / args.large_steps, 2), "iterations_per_step": iters,
                  "fp32_matvecs": gemv_n, "fp32_matvec_ms": round(gemv / max(gemv_n, 1), 4),
                  "device_bytes": dev}
+        if gemv_n and fmt == "theta":
+            entry["fp32_matvec_GBps"] = round(per32 / (gemv / gemv_n * 1e-3) / 1e9, 1)
         if half_n:
             per16 = per32 / 2 + float(M) * M * 4
             entry.update({"fp16_matvecs": half_n, "fp16_matvec_ms": round(half / half_n, 4),
@@ -491,7 +522,7 @@ def large_suspension(args):
             entry["speedup_vs_fp32_gmres"] = round(ref[2] / elapsed, 3)
             entry["pos_rel_err_vs_fp32_gmres"] = rel_err(p_end, ref[0])
             entry["ori_rel_err_vs_fp32_gmres"] = rel_err(o_end, ref[1])
-        out[solver.replace("-", "_")] = entry
+        out[key] = entry
     return out
 
 
@@ -619,7 +650,10 @@ def main():
     g["asm_flops"] = assembly_flops(args, args.solver, args.integration, pos, ori)
     M, K = args.fibers, args.steps
     value = M * K / g["elapsed"]
-    fmt = ("theta" if args.matrix_format in ("auto", "theta") else "dense") if args.solver in ITERATIVE else "dense"
+    if args.solver not in ITERATIVE or args.matrix_format == "dense":
+        fmt = "dense"
+    else:
+        fmt = "operator" if operator_form(args, args.solver) else "theta"
     line = {
         "metric": "fiber-steps/s at M=5000 (plain FP32 vs mixed-prec, pos err<=1e-6); p99 serve latency",
         "value": round(value, 2),
