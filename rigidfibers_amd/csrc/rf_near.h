@@ -190,8 +190,11 @@ __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_
       if (tid < PAIRS) smax[tid] = 0u;
       if (p < take) {
         const int j = js_[p];
-        float acc[NM][6];
-        inner_integrals<N, NQI, ANALYTIC>(xi, tid_, ti, sq_d, sq, pos[3 * j], pos[3 * j + 1], pos[3 * j + 2],
+        float acc[NM][6] = {};
+        // i itself is never listed: without this test the compiler's schedule of the
+        // exact integrals is slower (segments at M = 5000: 437 us, with it 391)
+        if (j != i)
+          inner_integrals<N, NQI, ANALYTIC>(xi, tid_, ti, sq_d, sq, pos[3 * j], pos[3 * j + 1], pos[3 * j + 2],
                                             ori[3 * j], ori[3 * j + 1], ori[3 * j + 2], pc, acc);
 #pragma unroll
         for (int m = 0; m < NM; ++m)
