@@ -197,7 +197,12 @@ RF_API void rf_destroy(rf_simulation* sim);
 
 /* Simulation::step(size_t) (src/simulation.cu:286-329): assemble, solve,
  * update velocities, update fibers (forward Euler when current_timestep == 0),
- * then rotate the state buffers. */
+ * then rotate the state buffers.  Where the near pairs only are stored
+ * (RF_MATRIX_AUTO above), their room is sized for 96 near sources per fiber at
+ * rf_create; an assembly that finds more waits for the device, allocates what
+ * they take and a quarter more in its place, and is repeated, or returns
+ * RF_ERR_OUT_OF_MEMORY (the state is unchanged, and there is no system until an
+ * assembly succeeds).  The room is not given back before rf_destroy. */
 RF_API rf_status rf_step(rf_simulation* sim, int64_t current_timestep);
 
 /* The four phases of Simulation::step, for VALIDATE-style dumps between them. */
@@ -245,7 +250,9 @@ RF_API int64_t rf_system_size(const rf_simulation* sim);
 
 RF_API rf_status rf_get_solver_stats(rf_simulation* sim, rf_solver_stats* stats);
 RF_API rf_status rf_get_timings(rf_simulation* sim, rf_timings* timings);
-/* Device bytes held by the simulation (admission accounting). */
+/* Device bytes held by the simulation (admission accounting).  With the near
+ * pairs only stored, they grow when a step finds more of them than there is
+ * room for (rf_step). */
 RF_API int64_t rf_device_bytes(const rf_simulation* sim);
 
 RF_API const char* rf_last_error(void);

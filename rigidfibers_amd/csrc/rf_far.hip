@@ -4,7 +4,7 @@
 // pair through its Q target nodes; for fibers whose centres lie far_rule's
 // radii apart (rf_device.h) the same projections follow from NP x NP kernel
 // values with NP = 6 or 8 (8 or 10 for N >= 6).  The near pairs are
-// assemble_theta_block's (rf_assemble.hip): both select by far_class, so every
+// assemble_near_block's (rf_near.h): both select by far_class, so every
 // pair is formed by exactly one of the two.
 //
 // Work decomposition.  Workgroup = one target fiber i, four wavefronts.  Each

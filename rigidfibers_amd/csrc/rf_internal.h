@@ -31,23 +31,26 @@ hipError_t launch_assemble_columns(int N, int NQI, bool analytical, int M, int64
                                    int jcount);
 hipError_t launch_sum_groups(int groups, int64_t len, const double* part, double* out, hipStream_t s);
 
-// Theta form (rf_assemble.hip): T holds NC = 3 + 6(N-1) component arrays of
+// Theta form (rf_theta.h): T holds NC = 3 + 6(N-1) component arrays of
 // stride Lp = theta_stride(M, N) per target fiber; *groups receives the number
 // of RHS partial slots written.  With Tv != nullptr it also stores the
 // velocity operator: 12 component arrays of the same stride per target fiber
 // (Theta_0 and Phi0 of every source mode) and the velocity constants
 // cpart[group][i][6] (cpart then holds max_pair_groups(M) * M * 6 doubles).
 PairGrid theta_grid(int M, int sources_per_iteration);
-// Below this many fibers one kernel forms every pair.  The launch is then
-// its latency, and the far kernel's own (24 us at M = 100: a few wavefronts with
-// one batch after another) is longer than what it takes off the near one's, or
-// saves little of a step: assembly in us, near alone / with the far kernel, at 0.1
-// fibers per unit volume: numerical M = 200 78 / 84, 250 107 / 95, 400 187 / 126;
-// analytical 300 103 / 124, 400 140 / 131, 600 243 / 196.  The lines lie above the
-// first gains: small suspensions are formed one way, bit for bit, since
-// trajectories through close contacts amplify the last bit of a system a
-// thousandfold and more.  A batch of 24 suspensions of 16 to 400 fibers (numerical)
-// takes 37.0 ms with no far pairs, 36.5 with those from 320 and 33.9 from 240.
+// Below this many fibers one kernel forms every pair.  The launch is then its
+// latency, and the far kernel's own is longer than what it saves, or saves little
+// of a step: warm assembly in us, every pair / far and near kernels, at 0.1 fibers
+// per unit volume: numerical M = 200 54 / 64, 250 77 / 73, 320 113 / 89, 400 165 /
+// 108, 600 346 / 176; exact 200 43 / 66, 320 86 / 91, 400 122 / 109, 448 143 / 126,
+// 600 241 / 178.  The lines lie somewhat above the first gains (13 us of a step of
+// 490 at M = 400 with exact integrals): the two ways differ in the last bits of a
+// system, which trajectories through close contacts amplify (10 steps of one batch,
+// numerical: 8.3e-7 from 64 bits with far pairs from 240 fibers, 1.5e-7 without;
+// other seeds not measured).  They are lines for one suspension: a served batch,
+// which fills the chip, takes 39.1 ms with no far pairs, 38.4 with these lines and
+// 33.5 with far pairs at every size (24 suspensions of 16 to 400 fibers, numerical;
+// 31.4 and 29.7 without and with them for exact integrals).
 __host__ __device__ constexpr int far_min_fibers(bool analytical) { return analytical ? 448 : 320; }
 // The far pairs (rf_far.hip): their sums go to the partial slots after the near
 // pairs' (slot0 on).

@@ -121,7 +121,7 @@ hipError_t gemv(const GemvPlan& p, const float* A, const double* x, double* part
 }
 
 // ---------------------------------------------------------------------------
-// y = A x with A in theta form (see rf_assemble.hip): for target fiber i
+// y = A x with A in theta form (see rf_theta.h): for target fiber i
 //   s0    = sum_{j,k_j} Q0_{ij,k_j} . x_{j,k_j}
 //   U_k   = sum_{j,k_j} Theta_{ij,k,k_j} x_{j,k_j}                  (k >= 1)
 //   y_i,0 = x_i,0 + D1 t_i s0

@@ -18,7 +18,8 @@ constexpr int kLuNb = 64;       // diagonal block: pivoting happens inside it
 constexpr int kLuPanel = 1024;  // outer panel
 // Panels per trailing update (its K = kLuGroup kLuPanel).  Measured at
 // n = 75 000 (BF16 ms per solve): 2 -> 528, 3 -> 404, 4 -> 405 (K = 4096; 3 takes
-// less memory); at n = 30 000 in FP32 1 -> 170, 2 -> 170, 3 -> 174.
+// less memory); at n = 30 000 in FP32 1 -> 170, 2 -> 170, 3 -> 174 (what
+// one rule for every mode costs there).
 constexpr int kLuGroup = 3;
 // The trailing update beside the look-ahead's panels (BF16 / FP16), once at
 // most kLuTailRows rows remain (where the panels' chain is the longer of the two):

@@ -26,9 +26,10 @@ namespace rf {
 // The self pair's columns are zeroed.  HALF (GMRES-IR's FP16 copy T16, S16):
 // phase 2 also takes each (target, source) block's largest |projection|,
 // phase 3 stores the block scales and the scaled FP16 values.
-// A suspension has few near sources (8 of 5000 in a ball at 0.028 fibers per
-// unit volume, about 20 at 0.1), so the sweeps are few and the scan, one
-// distance per source, is most of the launch.
+// Beside the far kernel a target has few near sources (8 of 5000 in a ball at 0.028
+// fibers per unit volume, about 20 at 0.1), so the sweeps are few and the scan, one
+// distance per source, is most of the launch.  SEGMENTS takes every source within
+// the first radius (46 and about 180 there).
 template <int N, int NQI, bool ANALYTIC, bool HALF = false, bool SEGMENTS = false>
 __device__ __forceinline__ void assemble_near_block(int i, int gy, int M, int64_t Lp, const double* __restrict__ pos,
                                                     const double* __restrict__ ori, float* __restrict__ T,

@@ -11,7 +11,7 @@
 // nodes, and its share of a product is
 //   g_i(s_p) += sum_q K(x_i + s_p t_i - x_j - s_q t_j) f_j(s_q),
 // f_j(s_q) = sum_m W_m(s_q) x_{j,m} formed once per source, the projections
-// TF_k = sum_p W_k(s_p) g_i(s_p) once per target: 960 instructions of a lane
+// TF_k = sum_p W_k(s_p) g_i(s_p) once per target: 926 instructions of a lane
 // per pair and no memory, 0.70 ms a product at M = 5000.  So far
 // pairs are not stored at all, the assembly forms only the others (46 of 5000
 // sources there, kept in theta form per target), and the right-hand side, the
@@ -88,8 +88,9 @@ __global__ void op_nodes_kernel(int M, int variant, const double* __restrict__ o
 // come through scalar registers.  With R = b_p - s_q t_j (b_p = x_i + s_p t_i -
 // x_j) and K f = a f + c (R . f) R, the sums over q are
 //   sum a_q f_q + b_p sum h_q - t_j sum s_q h_q,   h_q = c_q (b_p . f_q - s_q t_j . f_q):
-// two conversions and nine FP64 operations per kernel value, 960 instructions
-// per pair of fibers in all, issued in 97% of the slots (0.66 ms at M = 5000).
+// two conversions and nine FP64 operations per kernel value, 926 instructions
+// per pair of fibers in all, VALU instructions active in 98% of the cycles (counters;
+// 0.64 ms at M = 5000).
 // RHS = 2 sums two densities over the same kernel values (1.13 ms).  Tried:
 // centre differences kept in FP64 up to r^2 (0.70 ms) and the reciprocal square
 // root refined to FP64 (0.79 ms) left the system's error against FP64 where it

@@ -1,5 +1,5 @@
 // rf_pairs.h -- what the assembly kernels that form pairs by their target nodes
-// share (rf_assemble.hip, rf_near.h): the inner integrals of one pair at one
+// share (rf_assemble.hip, rf_theta.h, rf_near.h): the inner integrals of one pair at one
 // node, and the register budget.
 #pragma once
 

@@ -33,8 +33,8 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 
 // Every pair of one workgroup: target fiber i, source group gy.  For suspensions
-// below far_min_fibers and the direct solvers; the near kernel below, which lists
-// its sources, took 12 to 15% longer at this with exact integrals (M = 437: 147
+// below far_min_fibers and the direct solvers; the near kernel (rf_near.h), which
+// lists its sources, took 12 to 15% longer at this with exact integrals (M = 437: 147
 // against 130 us, 5000: 14.0 against 12.0 ms) and 2.5% with numerical ones in a
 // served batch (24 suspensions, 1.143 against 1.085 ms).
 //   phase 1  lane (p, q_i) writes G_m(q_i) of source slot p into LDS as row
